@@ -34,7 +34,9 @@ BLAS_SOURCES = ["blas.cpp"]
 # 128x128 tile copied every accumulator through VGPRs on each k slice.
 FILE_FLAGS = {"gemm_f64.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               # the grouped kernel's accumulators in VGPRs: 112 registers, four waves per SIMD
-              "grouped.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+              "grouped.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              # the solve kernels' small accumulators too (16 copies per slab otherwise)
+              "level3_kernels.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _compile(src: str) -> str:

@@ -52,6 +52,27 @@ struct Mfma<double> {
   __device__ static inline int col(int l) { return l & 15; }
 };
 
+// 16x16 blocks, four k per instruction: operand lane l -> (row / column l%16,
+// k l/16), accumulator r of lane l holds row row(r, l) of column l%16.
+template <typename T>
+struct Mfma16;
+template <>
+struct Mfma16<float> {  // v_mfma_f32_16x16x4_f32
+  using acc_t = floatx4;
+  __device__ static inline acc_t mma(float a, float b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  __device__ static inline int row(int r, int l) { return 4 * (l >> 4) + r; }
+};
+template <>
+struct Mfma16<double> {  // v_mfma_f64_16x16x4_f64
+  using acc_t = doublex4;
+  __device__ static inline acc_t mma(double a, double b, acc_t c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  __device__ static inline int row(int r, int l) { return (l >> 4) + 4 * r; }
+};
+
 __device__ inline float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ inline double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
@@ -94,6 +115,24 @@ __device__ inline double buf_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint3
   typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
   u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0);
   return __hiloint2double((int)v.y, (int)v.x);
+}
+
+// Workgroup barrier for data exchanged through LDS, which leaves global loads
+// in flight.  __syncthreads' release fence waits for every outstanding vector
+// memory operation (vmcnt(0)), including loads of slices or stages still
+// ahead, which cuts a load pipeline to one barrier interval.  Here each wave
+// waits for its own LDS operations only (lgkmcnt(0)): after the barrier every
+// wave's LDS writes are visible, and its LDS reads are complete, so a buffer
+// may be refilled.  A direct global-to-LDS load must have been waited for
+// (vmcnt) by the wave that issued it before the barrier that publishes it.
+// The empty asm statements' memory clobbers keep the compiler from moving LDS
+// reads or loads across it; the wait is the builtin so that the compiler's own
+// wait insertion sees it.
+__device__ inline void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt, expcnt unconstrained
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 // Map a linear workgroup id to a logical tile id so that each XCD (workgroups

@@ -128,23 +128,6 @@ __global__ void __launch_bounds__(256) pack_split_kernel(const float* __restrict
 
 __device__ inline void wait_vmcnt0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Barrier between LDS stages that leaves later stages' direct loads in
-// flight.  __syncthreads' release fence waits for every outstanding vector
-// memory operation (vmcnt(0)), including the direct-to-LDS loads of stages
-// still ahead, which cuts the pipeline to one stage in flight.  Here each
-// wave has already waited (vmcnt) for its own loads of the stage about to be
-// read, so after the barrier every wave's part of that stage is in LDS; its
-// own LDS reads of the previous stage are complete (lgkmcnt(0)) before it
-// arrives, so the buffer refilled next is free.  The empty asm statements'
-// memory clobbers keep the compiler from moving LDS reads or loads across
-// it; the wait is the builtin so that the compiler's own wait insertion
-// sees it.
-__device__ inline void stage_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt, expcnt unconstrained
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 template <int N>
 __device__ inline void wait_vmcnt() {
   // gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14
@@ -367,7 +350,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_split_packed_kernel(Split
 #pragma unroll
       for (int s = 0; s < NSTAGE; ++s) fill(s, s);
       wait_vmcnt<(NSTAGE - 1) * LPW>();
-      stage_barrier();
+      lds_barrier();
       u32x4 fa0[TERMS][RM], fb0[TERMS][RN], fa1[TERMS][RM], fb1[TERMS][RN];
       read_step(smem, 0, fa0, fb0);
       constexpr int NREAD = TERMS * (RM + RN), NMMA = (TERMS == 3 ? 6 : (TERMS == 2 ? 3 : 1)) * RM * RN;
@@ -379,7 +362,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_split_packed_kernel(Split
         __builtin_amdgcn_sched_barrier(0);
         // stage st + 1 must have landed; NSTAGE - 2 fills after it may not
         wait_vmcnt<(NSTAGE - 2) * LPW>();
-        stage_barrier();
+        lds_barrier();
         fill(st + NSTAGE, st % NSTAGE);
         // no LDS read is outstanding here (the barrier waited for them): this
         // wait costs nothing and keeps the compiler from counting the direct
@@ -405,7 +388,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_split_packed_kernel(Split
       // stage kt must have landed; the stages issued after it (at most
       // NSTAGE - 2, fewer near the end) may still be in flight
       wait_stages_behind<NSTAGE - 2, LPW>(nkt - 1 - kt);
-      stage_barrier();
+      lds_barrier();
       if (kt + NSTAGE - 1 < nkt) issue(kt + NSTAGE - 1, (kt + NSTAGE - 1) % NSTAGE);
       const unsigned char* base = smem + (kt % NSTAGE) * STAGE;
       u32x4 a[NSTEP][TERMS][RM], b[NSTEP][TERMS][RN];

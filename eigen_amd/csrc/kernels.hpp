@@ -83,11 +83,27 @@ struct TrtriParams {
 };
 template <typename T>
 hipError_t launch_trtri(const TrtriParams<T>& p, hipStream_t s);
-// D_p = [S_2p 0; 0 S_2p+1] (blocks of order L into blocks of order 2L,
-// off-diagonal blocks zero), p < count: the first step of doubling the
-// order of the inverted diagonal blocks.
+// One panel of a real triangular solve, in place: E X = alpha*B, E(i, k) = ta
+// ? A[k + i*lda] : A[i + k*lda] lower or upper of order sz <= kTrsmPanel, inv
+// its inverted diagonal blocks (launch_trtri), element (r, c) of the sz x
+// ncols right-hand sides at B[r*rs + c*cs].
+// lda <= kTrsmMaxLd keeps the offsets inside a 64-deep slab below 4 GB.
+constexpr int kTrsmPanel = 512;
+constexpr int64_t kTrsmMaxLd = 1 << 22;
 template <typename T>
-hipError_t launch_inverse_place(const T* S, T* D, int L, int64_t count, hipStream_t s);
+struct TrsmPanelParams {
+  const T* A;
+  const T* inv;
+  T* B;
+  int64_t lda, rs, cs;
+  int ta, lower, sz, ncols;
+  T alpha;
+};
+template <typename T>
+hipError_t launch_trsm_panel(const TrsmPanelParams<T>& p, hipStream_t s);
+// D (m x n, leading dimension m) = B.
+template <typename T>
+hipError_t launch_copy_block(const T* B, int64_t ldb, int m, int n, T* D, hipStream_t s);
 
 // Triangle of a complex rank update (level3_kernels.hip): on the lower
 // (upper) triangle, C = alpha*W + alpha2*f(W^T) + beta*C with f = conj when

@@ -10,9 +10,9 @@
 //   TRMM, TRSM     recursive 2x2 blocking of the triangle: at each level the
 //                  off-diagonal block is a plain product on the rest of B;
 //                  the leaves are products too (TRMM: the dense diagonal
-//                  block; TRSM: the inverse of the diagonal block, all of
-//                  them computed by one batched launch), so every flop but
-//                  the O(order * 64^2) of the inversions runs on MFMA.
+//                  block; complex TRSM: the inverse of the diagonal block,
+//                  all of them computed by one launch).  Real TRSM runs
+//                  panels of rows instead (trsm_panels).
 // Arguments are checked with the reference's rules (blas/level3_impl.h); the
 // BLAS wrappers in blas.cpp add the xerbla_ codes.
 //
@@ -68,20 +68,6 @@ eh_status zero_b(cplx<R>* B, int64_t m, int64_t n, int64_t ldb, hipStream_t s) {
   return e == hipSuccess ? EH_SUCCESS : hip_fail(e, "zero fill launch");
 }
 
-// order of the inverted diagonal blocks of TRSM
-template <typename T>
-constexpr int64_t trsm_leaf() {
-  return kTrsmLeaf;
-}
-template <>
-constexpr int64_t trsm_leaf<cplx<float>>() {
-  return kTrsmLeafComplex;
-}
-template <>
-constexpr int64_t trsm_leaf<cplx<double>>() {
-  return kTrsmLeafComplex;
-}
-
 // The triangular operator E = op(A) of order ka: E(i, k) = ta ? A[k + i*lda]
 // : A[i + k*lda]; `lower` is the triangle of E (the stored triangle of A
 // when not transposed, the other one when transposed).
@@ -105,18 +91,18 @@ int64_t half(int64_t sz, int64_t leaf) {
 }
 
 // ---- TRSM --------------------------------------------------------------------
-// The diagonal blocks of order trsm_leaf<T>() are inverted up front (one
-// launch), and for real types their order is then doubled up to
-// kTrsmLeafMax while it divides the order of the triangle: for every pair of
-// consecutive blocks at once (two batched products of the current order),
-//   lower:  inv([E11 0; E21 E22]) = [I1 0; -I2 E21 I1, I2]
-//   upper:  inv([E11 E12; 0 E22]) = [I1 -I1 E12 I2; 0 I2].
-// A leaf of the recursion multiplies its right-hand sides by the inverse of
-// its block, on the MFMA kernels, from a copy of them.  Larger leaves halve
-// the recursion's smallest and least efficient launches at each doubling
-// (a 64-row leaf multiplies 64 x n by 64 x 64).
-constexpr int64_t kTrsmLeafMax = 256;
-
+// Real types: the inverses of the 64 x 64 diagonal blocks (one launch), then
+// panels of kTrsmPanel rows in solve order, each one launch of the panel
+// kernel (level3_kernels.hip) and one product that takes it out of the rows
+// still to be solved.  Two launches per panel replace the recursion's one
+// product per block and level with a copy of every block: order 1000 with
+// 600 right-hand sides in FP64 took 58 launches and 372 us, against 6 and
+// 116 us.
+//
+// Complex types: the recursion below.  The diagonal blocks of order
+// kTrsmLeafComplex are inverted up front (one launch); a leaf of the
+// recursion multiplies its right-hand sides by the inverse of its block, on
+// the MFMA kernels, from a copy of them.
 template <typename T>
 struct IsCplx : std::false_type {};
 template <typename R>
@@ -129,32 +115,40 @@ struct TrsmWork {
   int64_t leaf;  // order of the inverted blocks
 };
 
+// E X = alpha*B (left) or X E = alpha*B (right) in place, real types; inv
+// holds the inverses of the diagonal blocks of E (left) or E^T (right).
 template <typename T>
-constexpr eh_dtype real_dtype() {
-  return std::is_same<T, double>::value ? EH_F64 : EH_F32;
-}
-
-// Inverses of order 2L in D (count = ka / 2L blocks) from those of order L in
-// S; tmp holds count blocks of order L.
-template <typename T>
-eh_status double_inverses(const Tri<T>& E, int64_t ka, int64_t L, const T* S, T* D, T* tmp, hipStream_t s) {
-  const int64_t count = ka / (2 * L), L2 = 2 * L;
-  hipError_t e = launch_inverse_place<T>(S, D, (int)L, count, s);
-  if (e != hipSuccess) return hip_fail(e, "inverse placement launch");
-  const int64_t sd = L2 * L2, st = L * L, se = L2 * (1 + E.lda);  // strides between pairs
-  const T one(1), zero(0), minus(-1);
-  constexpr eh_dtype dt = real_dtype<T>();
-  if (E.lower) {  // tmp = E21 I1; D(L:, :L) = -I2 tmp
-    EH_TRY(eh_gemm_batched_strided(dt, (eh_op)E.op(), EH_OP_N, L, L, L, &one, E.block(L, 0), E.lda, se, D, L2, sd,
-                                   &zero, tmp, L, st, count, s));
-    return eh_gemm_batched_strided(dt, EH_OP_N, EH_OP_N, L, L, L, &minus, D + L + L * L2, L2, sd, tmp, L, st, &zero,
-                                   D + L, L2, sd, count, s);
+eh_status trsm_panels(const Tri<T>& E, bool left, int64_t ka, int64_t other, T alpha, T* B, int64_t ldb, const T* inv,
+                      hipStream_t s) {
+  const bool lower = left ? E.lower : !E.lower;  // triangle of the operator that acts on columns
+  const int64_t np = (ka + kTrsmPanel - 1) / kTrsmPanel;
+  for (int64_t q = 0; q < np; ++q) {
+    const int64_t d = (lower ? q : np - 1 - q) * kTrsmPanel, sz = std::min<int64_t>(kTrsmPanel, ka - d);
+    T* Bp = left ? B + d : B + d * ldb;
+    TrsmPanelParams<T> p{};
+    p.A = E.diag(d);
+    p.inv = inv + d * kTrsmLeaf;
+    p.B = Bp;
+    p.lda = E.lda;
+    p.rs = left ? 1 : ldb;
+    p.cs = left ? ldb : 1;
+    p.ta = left ? E.ta : !E.ta;
+    p.lower = lower;
+    p.sz = (int)sz;
+    p.ncols = (int)other;
+    p.alpha = q == 0 ? alpha : T(1);
+    hipError_t e = launch_trsm_panel<T>(p, s);
+    if (e != hipSuccess) return hip_fail(e, "trsm panel launch");
+    // the rows still to be solved: below the panel (lower) or above it
+    const int64_t r0 = lower ? d + sz : 0, rows = lower ? ka - r0 : d;
+    if (rows == 0) continue;
+    const T beta = p.alpha;  // the first update scales the rest of B by alpha
+    if (left)
+      EH_TRY(prod(E.op(), EH_OP_N, rows, other, sz, T(-1), E.block(r0, d), E.lda, Bp, ldb, beta, B + r0, ldb, s));
+    else
+      EH_TRY(prod(EH_OP_N, E.op(), other, rows, sz, T(-1), Bp, ldb, E.block(d, r0), E.lda, beta, B + r0 * ldb, ldb, s));
   }
-  // tmp = E12 I2; D(:L, L:) = -I1 tmp
-  EH_TRY(eh_gemm_batched_strided(dt, (eh_op)E.op(), EH_OP_N, L, L, L, &one, E.block(0, L), E.lda, se, D + L + L * L2,
-                                 L2, sd, &zero, tmp, L, st, count, s));
-  return eh_gemm_batched_strided(dt, EH_OP_N, EH_OP_N, L, L, L, &minus, D, L2, sd, tmp, L, st, &zero, D + L * L2, L2,
-                                 sd, count, s);
+  return EH_SUCCESS;
 }
 
 // E[d:d+sz, d:d+sz] X = alpha*B, B = rows d.. of the right-hand sides (sz x n).
@@ -306,39 +300,39 @@ eh_status trsm_t(int side, int uplo, int transa, int diag, int64_t m, int64_t n,
   if (alpha == T(0)) return zero_b(B, m, n, ldb, s);
   if (!A) return fail(EH_ERR_INVALID, "A is NULL");
   const bool ta = transa != EH_OP_N;
-  const Tri<T> E{A, lda, ta, (uplo == EH_LOWER) != ta, diag == EH_UNIT, transa == EH_OP_C};
+  Tri<T> E{A, lda, ta, (uplo == EH_LOWER) != ta, diag == EH_UNIT, transa == EH_OP_C};
   const int64_t ka = side == EH_LEFT ? m : n;
-  constexpr int64_t leaf0 = trsm_leaf<T>();
-  // doubled leaf order (real types: the doubling runs on the batched
-  // product, which takes real operands)
-  int64_t leaf = leaf0;
-  if constexpr (!IsCplx<T>::value)
-    while (leaf < kTrsmLeafMax && ka % (2 * leaf) == 0) leaf *= 2;
-  const int64_t blocks0 = (ka + leaf0 - 1) / leaf0;
-  const int64_t inv0 = blocks0 * leaf0 * leaf0;                 // the inversion's blocks
-  const int64_t invd = leaf > leaf0 ? ka * leaf : 0;           // each doubled set (ka / L blocks of L^2)
-  const int64_t tmp = leaf > leaf0 ? ka * leaf / 4 : 0;        // (ka / 2L) blocks of L^2, L <= leaf / 2
-  const int64_t copy = side == EH_LEFT ? leaf * n : m * leaf;
+  constexpr int64_t leaf = IsCplx<T>::value ? kTrsmLeafComplex : kTrsmLeaf;
+  const int64_t blocks = (ka + leaf - 1) / leaf;
+  const int64_t inv = blocks * leaf * leaf;
+  const int64_t copy = !IsCplx<T>::value ? 0 : side == EH_LEFT ? leaf * n : m * leaf;
   StreamTemp t;
-  EH_TRY(t.get((size_t)(inv0 + 2 * invd + tmp + copy) * sizeof(T), s, "level-3 temporary"));
+  EH_TRY(t.get((size_t)(inv + copy) * sizeof(T), s, "level-3 temporary"));
   T* base = static_cast<T*>(t.ptr);
-  T* bufs[2] = {base + inv0, base + inv0 + invd};
-  T* tbuf = base + inv0 + 2 * invd;
-  TrtriParams<T> tp{A, lda, (int)E.ta, (int)E.lower, (int)E.unit, (int)ka, base};
+  StreamTemp dense;
+  if constexpr (!IsCplx<T>::value) {
+    if (lda > kTrsmMaxLd) {  // past the panel kernel's 32-bit offsets: a dense copy of the triangle
+      EH_TRY(dense.get((size_t)ka * ka * sizeof(T), s, "level-3 temporary"));
+      T* D = static_cast<T*>(dense.ptr);
+      hipError_t e = launch_tri_dense<T>(A, lda, (int)ka, D, ka, E.stored_lower(), false, E.unit, s);
+      if (e != hipSuccess) return hip_fail(e, "triangle expansion launch");
+      E.A = A = D;
+      E.lda = lda = ka;
+    }
+  }
+  // real types solve X E = alpha*B as E^T X^T = alpha*B^T
+  const bool flip = !IsCplx<T>::value && side == EH_RIGHT;
+  TrtriParams<T> tp{A, lda, (int)(E.ta != flip), (int)(E.lower != flip), (int)E.unit, (int)ka, base};
   tp.conj = E.conj;
   hipError_t e = launch_trtri<T>(tp, s);
   if (e != hipSuccess) return hip_fail(e, "diagonal block inversion launch");
-  const T* inv = base;
-  int which = 0;
   if constexpr (!IsCplx<T>::value) {
-    for (int64_t L = leaf0; L < leaf; L *= 2, which ^= 1) {
-      EH_TRY(double_inverses(E, ka, L, inv, bufs[which], tbuf, s));
-      inv = bufs[which];
-    }
+    return trsm_panels<T>(E, side == EH_LEFT, ka, side == EH_LEFT ? n : m, alpha, B, ldb, base, s);
+  } else {
+    const TrsmWork<T> w{base, base + inv, leaf};
+    return side == EH_LEFT ? trsm_left<T>(E, 0, m, B, ldb, n, alpha, w, s)
+                           : trsm_right<T>(E, 0, n, B, ldb, m, alpha, w, s);
   }
-  const TrsmWork<T> w{inv, tbuf + tmp, leaf};
-  return side == EH_LEFT ? trsm_left<T>(E, 0, m, B, ldb, n, alpha, w, s)
-                         : trsm_right<T>(E, 0, n, B, ldb, m, alpha, w, s);
 }
 
 template <typename T>

@@ -4,22 +4,22 @@
 // engine as GEMM (Eigen/src/Core/products/TriangularMatrixMatrix.h,
 // TriangularSolverMatrix.h, SelfadjointMatrixMatrix.h,
 // GeneralMatrixMatrixTriangular.h).  Here the bulk of their flops goes to the
-// MFMA product kernels through a recursive 2x2 blocking on the host; the two
-// kernels below do the rest:
+// MFMA product kernels through a blocking on the host; the kernels below do the
+// rest:
 //
 //   tri_dense_kernel   the dense form of a matrix stored in one triangle:
 //                      symmetric (mirror the stored triangle) or triangular
 //                      (zeros outside it, optional unit diagonal).  64x64
 //                      tiles; the mirrored half goes through LDS so that both
 //                      the reads and the writes are coalesced.  HBM-bound.
-//   trtri_kernel       the inverses of all 64 x 64 diagonal blocks of a
-//                      triangular matrix in one launch (one workgroup per
-//                      block, one thread per column of the inverse, the
-//                      column in registers, the block and the reciprocals of
-//                      its diagonal in LDS); the solve then multiplies each
-//                      diagonal block of right-hand sides by its inverse on
-//                      the MFMA kernels.
+//   trtri64_kernel     the inverses of all 64 x 64 diagonal blocks of a real
+//                      triangular matrix in one launch (trtri_kernel: the 32 x
+//                      32 blocks of a complex one);
+//   trsm_panel_kernel  the solve of up to 512 rows of a real system for 16
+//                      columns per workgroup, on those inverses.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -77,7 +77,319 @@ hipError_t launch_tri_dense(const T* A, int64_t lda, int n, T* D, int64_t ldd, b
   return hipGetLastError();
 }
 
-// Inverses of the diagonal blocks of a triangular matrix, one workgroup per
+// Inverses of the 64 x 64 diagonal blocks of a real triangular matrix, one
+// workgroup of four waves per block: block b is M_b(i, k) = mt ? A[k + i*lda]
+// : A[i + k*lda] at A + b*64 (1 + lda), of order nb = min(64, order - 64 b),
+// lower or upper, unit diagonal or not; its inverse goes to W + b*64*64
+// (ld 64, stored like M: column-major, or row-major when mt; zeros outside the
+// triangle).  Entries of M_b outside
+// its triangle and past nb are zero in LDS and the diagonal past nb is one.
+// An upper block is inverted as the lower one its reversed rows and columns
+// form.
+//
+// A block is a serial chain of 64 substitution steps, so latency bounds it.
+// Only its four 16 x 16 diagonal blocks are inverted by substitution, one wave
+// each, multiplying by the reciprocal of the diagonal as
+// TriangularSolverMatrix.h:67 does; the rest follows from
+//   inv([M11 0; M21 M22]) = [I1 0; -I2 (M21 I1), I2]
+// on the matrix cores, twice (16 -> 32 -> 64).  One thread per column of the
+// whole block (64 steps, 2048 unrolled multiply-adds) took 46.8 us for the 16
+// FP64 blocks of order 1000; this takes
+// 11.3 us.
+template <typename T>
+__global__ void __launch_bounds__(256) trtri64_kernel(TrtriParams<T> p) {
+  using F = Mfma16<T>;
+  constexpr int NB = 64;
+  __shared__ T M[NB][NB + 1], V[NB][NB + 1], P[NB][33];
+  __shared__ T dinv[NB];
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nb = min(NB, p.order - b * NB);
+  const T* A = p.A + (int64_t)b * NB * (1 + p.lda);
+  const bool rev = !p.lower;
+#pragma unroll
+  for (int q = 0; q < NB * NB / 256; ++q) {  // lanes walk the contiguous index of A
+    const int c = lane, o = w + 4 * q;
+    const int i = p.mt ? o : c, k = p.mt ? c : o;
+    const bool in = i < nb && k < nb && (p.lower ? k < i : k > i);
+    const T x = in ? A[c + (int64_t)o * p.lda] : T(0);
+    M[rev ? NB - 1 - i : i][rev ? NB - 1 - k : k] = x;
+    V[o][c] = T(0);
+  }
+  if (tid < NB) dinv[rev ? NB - 1 - tid : tid] = (tid >= nb || p.unit) ? T(1) : recip(A[tid + (int64_t)tid * p.lda]);
+  __syncthreads();
+  {  // 16 x 16 diagonal blocks: lane v < 16 of wave w solves for column v of block w
+    const int o = 16 * w, v = lane & 15;
+    T x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = i == v ? T(1) : T(0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      x[i] *= dinv[o + i];
+#pragma unroll
+      for (int r = i + 1; r < 16; ++r) x[r] = fma_t(-M[o + r][o + i], x[i], x[r]);
+    }
+    if (lane < 16) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) V[o + i][o + v] = x[i];
+    }
+  }
+  __syncthreads();
+  const int li = lane & 15, lg = lane >> 4;
+  // 16 x 16 block of X*Y over K terms, X and Y given by element functions
+  auto product = [&](int K, auto x, auto y) {
+    typename F::acc_t acc;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = T(0);
+#pragma unroll
+    for (int k = 0; k < K; k += 4) acc = F::mma(x(li, k + lg), y(k + lg, li), acc);
+    return acc;
+  };
+  // 16 -> 32: waves 0 and 1 take the two pairs of blocks
+  const int o = 32 * (w & 1);
+  if (w < 2) {
+    const auto t = product(16, [&](int i, int k) { return M[o + 16 + i][o + k]; }, [&](int k, int j) { return V[o + k][o + j]; });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) P[o + F::row(r, lane)][li] = t[r];
+  }
+  __syncthreads();
+  if (w < 2) {
+    const auto t = product(16, [&](int i, int k) { return V[o + 16 + i][o + 16 + k]; }, [&](int k, int j) { return P[o + k][j]; });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) V[o + 16 + F::row(r, lane)][o + li] = -t[r];
+  }
+  __syncthreads();
+  // 32 -> 64: the 32 x 32 off-diagonal block, one 16 x 16 quarter per wave
+  const int ti = 16 * (w & 1), tj = 16 * (w >> 1);
+  {
+    const auto t = product(32, [&](int i, int k) { return M[32 + ti + i][k]; }, [&](int k, int j) { return V[k][tj + j]; });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) P[ti + F::row(r, lane)][tj + li] = t[r];
+  }
+  __syncthreads();
+  {
+    const auto t = product(32, [&](int i, int k) { return V[32 + ti + i][32 + k]; }, [&](int k, int j) { return P[k][tj + j]; });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) V[32 + ti + F::row(r, lane)][tj + li] = -t[r];
+  }
+  __syncthreads();
+  T* W = p.W + (int64_t)b * NB * NB;
+#pragma unroll
+  for (int q = 0; q < NB * NB / 256; ++q) {
+    const int i = lane, k = w + 4 * q;
+    // p.mt: row i of the inverse is contiguous in W, else column k
+    const int r = p.mt ? k : i, c = p.mt ? i : k;
+    W[i + k * NB] = rev ? V[NB - 1 - r][NB - 1 - c] : V[r][c];
+  }
+}
+
+// Solve of one panel of a real triangular system in place: E X = alpha*B with
+// E of order sz (lower or upper, E(i, k) = ta ? A[k + i*lda] : A[i + k*lda])
+// and B's element (r, c) at B[r*rs + c*cs].  Columns are independent, so a
+// workgroup takes 16 of them and holds them in LDS for the whole solve; E
+// streams from the caches once per workgroup.  Per 64-row block b (in solve
+// order)
+//   Y = B_b - sum_{j solved} E(b, j) X_j,   X_b = inv(E_bb) Y
+// as 16-row strips of 16x16x4 MFMAs.
+//
+// What bounds it: the chain of blocks, two dependent 64-deep products and
+// three barriers each, and the matrix cores of the ceil(ncols / 16) CUs in
+// use.  Sixteen waves, four per strip (and SIMD): the waves of group 0 run the
+// chain -- E(b, b-1) X_(b-1), then the inverse -- while groups 1 to 3 share
+// the products with the blocks solved earlier, one block ahead of the chain,
+// so its latencies are filled with their MFMAs.  E does not depend on the
+// solve: every wave loads its next 64-deep slab (16 values per lane) before it
+// multiplies the current one, and the barriers wait for LDS only.
+// A 512-row FP64 panel with 600 columns takes 38.5 us (15.4 us of MFMA issue on
+// 38 CUs); with one group of waves and three slabs ahead in registers it took
+// 52 us.
+template <typename T, bool TA>
+__global__ void __launch_bounds__(1024) trsm_panel_kernel(TrsmPanelParams<T> p) {
+  using F = Mfma16<T>;
+  constexpr int NB = kTrsmLeaf, NC = 16, XS = NC + 1, NT = 1024, NH = 3;  // NH: helper groups
+  constexpr int EPC = 16 / sizeof(T);  // consecutive k of one lane
+  __shared__ T Xs[kTrsmPanel * XS];    // row r of the panel at Xs[r*XS]
+  __shared__ T Y[NB * XS];
+  __shared__ T R[NH][NB * XS];         // partial sums of the helper groups
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int strip = w & 3, group = w >> 2;
+  const int li = lane & 15, lg = lane >> 4;
+  const int c0 = blockIdx.x * NC;
+  const int nblk = (p.sz + NB - 1) / NB;
+  T* B = p.B + c0 * p.cs;
+  const int nc = min(NC, p.ncols - c0);
+  auto blk = [&](int s) { return p.lower ? s : nblk - 1 - s; };  // block solved at step s
+
+  // slab of E or of an inverse: lane's values v[q*EPC + e] = X(16 strip + li, k)
+  // with k = 4*EPC*q + EPC*lg + e, q < 16 / EPC
+  struct Slab {
+    T v[16];
+  };
+  // The slab of E(blk(s), blk(j)), or of the inverse of block blk(s) when j <
+  // 0, through a buffer resource based at the slab, so that a load costs one
+  // scalar add.  Reads past the panel's last element return zero.
+  const uint32_t vo_e = (uint32_t)((TA ? (int64_t)li * p.lda + EPC * lg : (int64_t)EPC * lg * p.lda + li) * sizeof(T));
+  const uint32_t vo_i = (uint32_t)((TA ? li * NB + EPC * lg : EPC * lg * NB + li) * sizeof(T));
+  auto load = [&](int s, int j) {
+    Slab t;
+    const bool inv = j < 0;
+    const int64_t ld = inv ? NB : p.lda;
+    const int i0 = (inv ? 0 : blk(s) * NB) + 16 * strip, k0 = inv ? 0 : blk(j) * NB, end = inv ? NB : p.sz;
+    const int64_t first = TA ? k0 + i0 * ld : i0 + k0 * ld, last = (end - 1) * (ld + 1);
+    const T* base = (inv ? p.inv + (int64_t)blk(s) * NB * NB : p.A) + first;
+    const __amdgpu_buffer_rsrc_t rs =
+        make_rsrc(base, (uint32_t)max((int64_t)0, min((last - first + 1) * (int64_t)sizeof(T), (int64_t)0xFFFFFFF0)));
+    const uint32_t vo = inv ? vo_i : vo_e;
+    if constexpr (TA) {
+#pragma unroll
+      for (int q = 0; q < 16 / EPC; ++q)
+        *reinterpret_cast<u32x4*>(&t.v[q * EPC]) = buf_load16(rs, vo, 4 * EPC * q * sizeof(T));
+    } else {
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        t.v[q] = buf_load(rs, vo, (uint32_t)((4 * EPC * (q / EPC) + q % EPC) * ld * sizeof(T)), (T*)nullptr);
+    }
+    return t;
+  };
+  // acc + slab * x, x the 64 rows of LDS at `x`; k0: the slab's first column
+  // of the panel (-NB: an inverse).  k-contiguous rows run on into the next
+  // row past the panel's last column (the ragged last block of an upper
+  // panel): zeros from there on.
+  struct Acc {
+    typename F::acc_t a, b;
+  };
+  auto multiply = [&](const Slab& t, const T* x, int k0, Acc& acc) {
+    const int live = p.sz - max(k0, 0) - EPC * lg;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int k = 4 * EPC * (q / EPC) + q % EPC;
+      const T a = !TA || k0 < 0 || k < live ? t.v[q] : T(0);
+      const T y = x[(k + EPC * lg) * XS + li];
+      if (q & 1)
+        acc.b = F::mma(a, y, acc.b);
+      else
+        acc.a = F::mma(a, y, acc.a);
+    }
+  };
+  auto clear = [&](Acc& acc) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc.a[r] = acc.b[r] = T(0);
+  };
+
+  // panel -> LDS, threads along the contiguous index of B; zeros past sz and nc
+  const bool rows_fast = p.rs == 1;
+  const int rows = nblk * NB, total = rows * NC;
+  auto fill = [&]() {
+    for (int q = tid; q < total; q += NT) {
+      const int r = rows_fast ? q % rows : q / NC, c = rows_fast ? q / rows : q % NC;
+      Xs[r * XS + c] = r < p.sz && c < nc ? p.alpha * B[r * p.rs + c * p.cs] : T(0);
+    }
+  };
+  // Both branches run the same barriers: one after the fill, three per step.
+  if (group == 0) {
+    __builtin_amdgcn_s_setprio(3);  // the chain's MFMAs go before the helpers'
+    Slab inv = load(0, -1), sub = load(min(1, nblk - 1), 0);
+    fill();
+    lds_barrier();
+    Acc acc;
+    for (int s = 0; s < nblk; ++s) {
+      const int b = blk(s), nx = min(s + 1, nblk - 1);
+      clear(acc);
+      if (s > 0) multiply(sub, Xs + blk(s - 1) * NB * XS, blk(s - 1) * NB, acc);
+      if (s > 0) sub = load(nx, s);
+      lds_barrier();  // the helpers' sums are in R
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * strip + F::row(r, lane), o = row * XS + li;
+        T v = Xs[b * NB * XS + o] - (acc.a[r] + acc.b[r]);
+        if (s > 1) v -= (R[0][o] + R[1][o]) + R[2][o];
+        Y[o] = b * NB + row < p.sz ? v : T(0);
+      }
+      lds_barrier();  // Y
+      clear(acc);
+      multiply(inv, Y, -NB, acc);
+      inv = load(nx, -1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Xs[(b * NB + 16 * strip + F::row(r, lane)) * XS + li] = acc.a[r] + acc.b[r];
+      lds_barrier();  // X of block b
+    }
+  } else {
+    // E(s, j) for j = group - 1, group + 2, ... < s - 1, s = 2 ...
+    int ns = group + 1, nj = group - 1;  // the next slab to load
+    auto load_next = [&]() {
+      const Slab t = load(min(ns, nblk - 1), min(nj, nblk - 1));
+      nj += NH;
+      if (nj >= ns - 1) {
+        ++ns;
+        nj = group - 1;
+      }
+      return t;
+    };
+    Slab next = load_next();
+    fill();
+    lds_barrier();
+    Acc acc;
+    clear(acc);
+    int j = group - 1;  // the next product of the step ahead
+    auto product = [&]() {
+      const Slab cur = next;
+      next = load_next();
+      multiply(cur, Xs + blk(j) * NB * XS, blk(j) * NB, acc);
+      j += NH;
+    };
+    for (int s = 0; s < nblk; ++s) {
+      while (j < s - 1) product();
+      if (s > 1) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) R[group - 1][(16 * strip + F::row(r, lane)) * XS + li] = acc.a[r] + acc.b[r];
+      }
+      lds_barrier();  // R
+      lds_barrier();  // Y
+      clear(acc);
+      j = group - 1;
+      if (j < s && s + 1 < nblk) product();  // blocks before s are solved
+      lds_barrier();  // X of block blk(s)
+    }
+  }
+  for (int q = tid; q < total; q += NT) {
+    const int r = rows_fast ? q % rows : q / NC, c = rows_fast ? q / rows : q % NC;
+    if (r < p.sz && c < nc) B[r * p.rs + c * p.cs] = Xs[r * XS + c];
+  }
+}
+
+template <typename T>
+hipError_t launch_trsm_panel(const TrsmPanelParams<T>& p, hipStream_t s) {
+  if (p.sz <= 0 || p.ncols <= 0) return hipSuccess;
+  if (p.sz > kTrsmPanel) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)((p.ncols + 15) / 16));
+  if (p.ta)
+    hipLaunchKernelGGL((trsm_panel_kernel<T, true>), grid, dim3(1024), 0, s, p);
+  else
+    hipLaunchKernelGGL((trsm_panel_kernel<T, false>), grid, dim3(1024), 0, s, p);
+  return hipGetLastError();
+}
+template hipError_t launch_trsm_panel<float>(const TrsmPanelParams<float>&, hipStream_t);
+template hipError_t launch_trsm_panel<double>(const TrsmPanelParams<double>&, hipStream_t);
+
+// D (m x n, ld m) = B: one thread per element, lanes along the columns' rows.
+template <typename T>
+__global__ void __launch_bounds__(256) copy_block_kernel(const T* B, int64_t ldb, int m, int64_t total, T* D) {
+  for (int64_t idx = blockIdx.x * 256ll + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256)
+    D[idx] = B[idx % m + idx / m * ldb];
+}
+template <typename T>
+hipError_t launch_copy_block(const T* B, int64_t ldb, int m, int n, T* D, hipStream_t s) {
+  const int64_t total = (int64_t)m * n;
+  if (total <= 0) return hipSuccess;
+  const int64_t blocks = std::min<int64_t>((total + 255) / 256, 4096);
+  hipLaunchKernelGGL(copy_block_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, s, B, ldb, m, total, D);
+  return hipGetLastError();
+}
+template hipError_t launch_copy_block<float>(const float*, int64_t, int, int, float*, hipStream_t);
+template hipError_t launch_copy_block<double>(const double*, int64_t, int, int, double*, hipStream_t);
+
+// The same for complex types, blocks of order NB, one workgroup per
 // block: block b is M_b(i, k) = mt ? A[k + i*lda] : A[i + k*lda] at A + b*NB
 // (1 + lda), of order nb = min(NB, order - b*NB), lower or upper, unit
 // diagonal or not.  Thread v solves M_b x = e_v by substitution, multiplying
@@ -86,8 +398,8 @@ hipError_t launch_tri_dense(const T* A, int64_t lda, int n, T* D, int64_t ldd, b
 // outside the triangle and past nb).  Entries of M_b outside its triangle
 // and past nb are zero in LDS and the reciprocal diagonal past nb is one, so
 // the unrolled substitution needs no guards.  Each dot product runs as two
-// interleaved partial sums (half the dependent chain).  T is a real type or
-// cplx<R> (then p.conj conjugates M, for an inverse of A^H's blocks).
+// interleaved partial sums (half the dependent chain).  p.conj conjugates M,
+// for an inverse of A^H's blocks.
 template <typename T, int NB>
 __global__ void __launch_bounds__(NB) trtri_kernel(TrtriParams<T> p) {
   __shared__ T M[NB][NB];
@@ -197,54 +509,28 @@ template hipError_t launch_tri_combine<double>(const cplx<double>*, int64_t, int
                                                cplx<double>, cplx<double>, bool, cplx<double>, bool, hipStream_t);
 
 template <typename T>
-struct TrsmLeafOf {
-  static constexpr int value = kTrsmLeaf;
+struct TrtriLaunch {  // real types
+  static constexpr int NB = kTrsmLeaf, NT = 256;
+  static constexpr auto kernel = trtri64_kernel<T>;
 };
 template <typename R>
-struct TrsmLeafOf<cplx<R>> {
-  static constexpr int value = kTrsmLeafComplex;
+struct TrtriLaunch<cplx<R>> {
+  static constexpr int NB = kTrsmLeafComplex, NT = kTrsmLeafComplex;
+  static constexpr auto kernel = trtri_kernel<cplx<R>, kTrsmLeafComplex>;
 };
 
 template <typename T>
 hipError_t launch_trtri(const TrtriParams<T>& p, hipStream_t s) {
   if (p.order <= 0) return hipSuccess;
-  constexpr int NB = TrsmLeafOf<T>::value;
-  const unsigned blocks = (unsigned)((p.order + NB - 1) / NB);
-  hipLaunchKernelGGL((trtri_kernel<T, NB>), dim3(blocks), dim3(NB), 0, s, p);
-  return hipGetLastError();
-}
-
-// D_p = [S_2p 0; 0 S_2p+1] for p < count: S holds 2*count blocks of order
-// L (L x L, column-major, consecutive), D count blocks of order 2L; the
-// off-diagonal blocks are zeroed (one of them is then overwritten by the
-// doubling product).  One thread per element of D.
-template <typename T>
-__global__ void __launch_bounds__(256) inverse_place_kernel(const T* __restrict__ S, T* __restrict__ D, int L,
-                                                            int64_t total) {
-  const int64_t idx = blockIdx.x * 256ll + threadIdx.x;
-  if (idx >= total) return;
-  const int64_t blk = 4ll * L * L;
-  const int64_t p = idx / blk, r = idx % blk;
-  const int j = (int)(r / (2 * L)), i = (int)(r % (2 * L));
-  T v = T(0);
-  if (i < L && j < L) v = S[(2 * p) * L * L + i + (int64_t)j * L];
-  if (i >= L && j >= L) v = S[(2 * p + 1) * L * L + (i - L) + (int64_t)(j - L) * L];
-  D[idx] = v;
-}
-
-template <typename T>
-hipError_t launch_inverse_place(const T* S, T* D, int L, int64_t count, hipStream_t s) {
-  const int64_t total = count * 4ll * L * L;
-  if (total <= 0) return hipSuccess;
-  hipLaunchKernelGGL(inverse_place_kernel<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, S, D, L, total);
+  using L = TrtriLaunch<T>;
+  hipLaunchKernelGGL(L::kernel, dim3((unsigned)((p.order + L::NB - 1) / L::NB)), dim3(L::NT), 0, s, p);
   return hipGetLastError();
 }
 
 #define EH_L3_INST(T)                                                                                       \
   template hipError_t launch_tri_dense<T>(const T*, int64_t, int, T*, int64_t, bool, bool, bool, hipStream_t, \
                                           bool, bool);                                                      \
-  template hipError_t launch_trtri<T>(const TrtriParams<T>&, hipStream_t);                                  \
-  template hipError_t launch_inverse_place<T>(const T*, T*, int, int64_t, hipStream_t);
+  template hipError_t launch_trtri<T>(const TrtriParams<T>&, hipStream_t);
 EH_L3_INST(float)
 EH_L3_INST(double)
 EH_L3_INST(cplx<float>)
