@@ -133,6 +133,7 @@ int plan_packed(int kind, int opa, int opb, int64_t m, int64_t n, int64_t k) {
 }
 
 bool mlp_has_default();
+bool mlp_installed();
 
 static std::mutex g_mutex;
 static int g_mode = -1;  // -1: not yet chosen (EIGEN_AMD_TUNE, else MLP when compiled in)
@@ -167,7 +168,21 @@ struct WorkspaceSlot {
 static std::map<std::tuple<int, hipStream_t, std::thread::id>, std::unique_ptr<WorkspaceSlot>> g_ws;
 
 Workspace::~Workspace() {
-  if (ptr) (void)hipFree(ptr);
+  if (base) (void)hipFree(base);
+}
+
+// Tickets of the balanced products, zero between calls: cleared when the
+// buffer first serves one (the caller's stream is not being captured), and
+// by the last taker of each from then on.
+static eh_status workspace_tickets(hipStream_t stream, WorkspaceLease& lease, unsigned** tickets) {
+  Workspace& w = *lease.buf;
+  if (!w.tickets_clear) {
+    hipError_t e = hipMemsetAsync(w.base, 0, kTicketBytes, stream);
+    if (e != hipSuccess) return hip_fail(e, "ticket clear");
+    w.tickets_clear = true;
+  }
+  *tickets = static_cast<unsigned*>(w.base);
+  return EH_SUCCESS;
 }
 
 static thread_local void* t_fixed_ptr = nullptr;
@@ -209,11 +224,12 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
     auto fresh = std::make_shared<Workspace>();
     const size_t want = std::max(bytes, std::max(have, (size_t)1 << 20));
     slot->buf.reset();  // the old buffer goes once no lease refers to it
-    e = hipMalloc(&fresh->ptr, want);
+    e = hipMalloc(&fresh->base, want + kTicketBytes);
     if (e != hipSuccess) {
-      fresh->ptr = nullptr;
+      fresh->base = nullptr;
       return fail(EH_ERR_ALLOC, std::string("hipMalloc(workspace): ") + hipGetErrorString(e));
     }
+    fresh->ptr = static_cast<unsigned char*>(fresh->base) + kTicketBytes;
     fresh->bytes = want;
     slot->buf = std::move(fresh);
   }
@@ -440,6 +456,26 @@ static eh_status launch_bf16_product(bool ta, bool tb, int m, int n, int k, floa
 }
 
 template <typename T>
+static GemmParams<T> product_params(bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha, const T* A, int64_t lda,
+                                    const T* B, int64_t ldb, T beta, T* C, int64_t ldc) {
+  GemmParams<T> p{};
+  p.A = A;
+  p.B = B;
+  p.C = C;
+  p.lda = lda;
+  p.ldb = ldb;
+  p.ldc = ldc;
+  p.M = (int)m;
+  p.N = (int)n;
+  p.K = (int)k;
+  p.alpha = alpha;
+  p.beta = beta;
+  p.bytesA = (uint32_t)((ta ? (uint64_t)(m - 1) * lda + k : (uint64_t)(k - 1) * lda + m) * sizeof(T));
+  p.bytesB = (uint32_t)((!tb ? (uint64_t)(n - 1) * ldb + k : (uint64_t)(k - 1) * ldb + n) * sizeof(T));
+  return p;
+}
+
+template <typename T>
 static eh_status launch_product(bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha, const T* A,
                                 int64_t lda, const T* B, int64_t ldb, T beta, T* C, int64_t ldc, bool split_prec,
                                 int terms, int config, hipStream_t stream, int tri = 0) {
@@ -478,21 +514,8 @@ static eh_status launch_product(bool ta, bool tb, int64_t m, int64_t n, int64_t 
     return fail(EH_ERR_UNSUPPORTED, "operand leading dimension too large for 32-bit addressing");
   }
 
-  GemmParams<T> p{};
-  p.A = A;
-  p.B = B;
-  p.C = C;
-  p.lda = lda;
-  p.ldb = ldb;
-  p.ldc = ldc;
-  p.M = (int)m;
-  p.N = (int)n;
-  p.K = (int)k;
-  p.alpha = alpha;
-  p.beta = beta;
+  GemmParams<T> p = product_params<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
   p.tri = tri;
-  p.bytesA = (uint32_t)((ta ? (uint64_t)(m - 1) * lda + k : (uint64_t)(k - 1) * lda + m) * sizeof(T));
-  p.bytesB = (uint32_t)((!tb ? (uint64_t)(n - 1) * ldb + k : (uint64_t)(k - 1) * ldb + n) * sizeof(T));
 
   int tile = 0, splits = 1, kslice = (int)(128 / sizeof(T));
   hipError_t e;
@@ -530,6 +553,136 @@ static eh_status launch_product(bool ta, bool tb, int64_t m, int64_t n, int64_t 
   }
   return EH_SUCCESS;
 }
+
+// Launches p on the balanced kernel: with tickets and slots from the stream's
+// workspace or the installed fixed scratch, or (one workgroup per tile)
+// without, in a captured call: it may be replayed beside other work of this
+// stream's workspace.  (A plain product then keeps its configuration, run_gemm
+// below.)
+static bool balanced_workspace_allowed(hipStream_t stream) {
+  if (fixed_scratch_active()) return true;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return cap == hipStreamCaptureStatusNone;
+}
+
+// Workgroups the balanced kernel runs: it fits three to a CU, and short runs
+// do better as two longer ones (FP64 1000x777x1203, 62 slices per CU: 50.1
+// against 50.6 us; FP32 726x2066x1032, 51: 41.8 against 44.1; FP64
+// 2048x700x3000, 258: 164 against 159).
+constexpr int kCUs = 256;
+static int balanced_groups(int64_t units) {
+  int64_t g = kCUs * (units < 120 * kCUs ? 2 : 3);
+  while (g > 8 && units < 4 * g) g /= 2;  // at least four slices each
+  return (int)std::min(g, units);
+}
+
+template <typename T>
+eh_status launch_balanced(GemmParams<T> p, int mode, bool ta, bool tb, hipStream_t stream,
+                          size_t min_workspace = 0) {
+  int64_t tiles = 0, units = 0;
+  balanced_extent<T>(p, mode, &tiles, &units);
+  WorkspaceLease lease;
+  unsigned* tickets = nullptr;
+  int groups = 0;
+  if (tiles <= (int64_t)(kTicketBytes / 4) && balanced_workspace_allowed(stream)) {
+    groups = balanced_groups(units);
+    constexpr int b = kBalancedTile;
+    void* ws = nullptr;
+    const size_t slots = (size_t)groups * 2 * b * b * sizeof(T);
+    if (fixed_scratch_active()) {
+      // nothing in the fixed scratch outlives a call: the tickets lie behind
+      // the slots and are cleared first (a kernel, so a capture may hold it)
+      eh_status st = workspace_get(stream, slots + (size_t)tiles * sizeof(unsigned), &lease, &ws);
+      if (st != EH_SUCCESS) return st;
+      tickets = reinterpret_cast<unsigned*>(static_cast<unsigned char*>(ws) + slots);
+      hipError_t e = launch_scale_c<float>(reinterpret_cast<float*>(tickets), (int)tiles, 1, tiles, 0.0f, stream);
+      if (e != hipSuccess) return hip_fail(e, "ticket clear launch");
+    } else if (workspace_get(stream, std::max(slots, min_workspace), &lease, &ws) != EH_SUCCESS ||
+               workspace_tickets(stream, lease, &tickets) != EH_SUCCESS) {
+      (void)hipGetLastError();  // no room for the slots: one workgroup per tile needs none
+      groups = 0;
+    }
+    p.W = static_cast<T*>(ws);
+  }
+  KernelTimer t(EH_KC_PRODUCT, stream);
+  hipError_t e = launch_gemm_balanced<T>(p, mode, ta, tb, groups, tickets, stream);
+  return e == hipSuccess ? EH_SUCCESS : hip_fail(e, "balanced product launch");
+}
+
+// Enough 128x128 tiles that the planner's kernels with their larger tiles are
+// the faster ones (FP64 4096^3: 2.08 against 2.26 ms, FP32 4096^3: 1.02 against
+// 1.13).
+static bool many_large_tiles(bool f64, int64_t m, int64_t n) {
+  return ((m + 127) / 128) * ((n + 127) / 128) >= (f64 ? 2 : 1) * kCUs;
+}
+
+// Whether a plain product leaves configuration `config` for the balanced
+// kernel.  With `work` the time of the padded product at
+// three quarters of the peak, the configuration loses the idle part of its
+// last round of workgroups and, when it splits K, a reduction launch and its
+// traffic; the balanced kernel loses a few us, and a share of its time, to cut
+// tiles.  Measured, configuration against balanced: FP64 2874x1426x1995 336 /
+// 290 us, 2048x700x3000 187 / 159, 1573x721x1984 109 / 104, 1000x777x1203 56 /
+// 50; FP32 1645x1384x2732 132 / 123, 779x796x1129 33 / 25; on the other side
+// FP64 2887x1224x505 75 / 83, 2629x660x760 60 / 63, FP32 2801x2411x710 96 / 106.
+static bool balanced_pays(bool f64, int64_t m, int64_t n, int64_t k, int config) {
+  if (many_large_tiles(f64, m, n)) return false;
+  int tile, splits;
+  config_decode(config, &tile, &splits);
+  auto count = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  const int64_t wgs = count(kTileM[tile], kTileN[tile]) * splits;
+  const double idle = (double)((wgs + kCUs - 1) / kCUs * kCUs) / (double)wgs - 1.0;
+  const double flops_per_us = f64 ? 59e6 : 118e6;
+  const double work = 2.0 * (double)(count(64, 64) * 4096) * (double)k / flops_per_us;
+  const double reduce = splits > 1 ? 2.0 + (double)splits * (double)m * (double)n * (f64 ? 8 : 4) / 4e6 : 0.0;
+  return idle * work + reduce >= (f64 ? 10.0 + 0.06 * work : 4.0 + 0.10 * work);
+}
+
+template <typename T>
+bool tri_product(bool left, bool tri_t, bool lower, bool unit, int64_t order, int64_t other, T alpha, const T* E,
+                 int64_t lde, const T* X, int64_t ldx, T* C, int64_t ldc, hipStream_t stream, eh_status* st) {
+  const bool ta = left && tri_t, tb = !left && tri_t;
+  const int64_t m = left ? order : other, n = left ? other : order;
+  const T* A = left ? E : X;
+  const T* B = left ? X : E;
+  const int64_t lda = left ? lde : ldx, ldb = left ? ldx : lde;
+  if (!operand_fits<T>(ta, m, order, lda) || !operand_fits<T>(!tb, n, order, ldb)) return false;
+  GemmParams<T> p = product_params<T>(ta, tb, m, n, order, alpha, A, lda, B, ldb, T(0), C, ldc);
+  p.lower = lower;
+  p.unit = unit;
+  *st = launch_balanced<T>(p, left ? kTriA : kTriB, ta, tb, stream);
+  return true;
+}
+template bool tri_product<float>(bool, bool, bool, bool, int64_t, int64_t, float, const float*, int64_t, const float*,
+                                 int64_t, float*, int64_t, hipStream_t, eh_status*);
+template bool tri_product<double>(bool, bool, bool, bool, int64_t, int64_t, double, const double*, int64_t,
+                                  const double*, int64_t, double*, int64_t, hipStream_t, eh_status*);
+
+template <typename T>
+bool complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,
+                       const T* B3, int64_t ldb3, T beta, T* C, int64_t ldc, int prec, hipStream_t stream,
+                       eh_status* st) {
+  if (std::is_same<T, float>::value && prec == EH_PREC_AUTO) prec = default_sgemm_precision();
+  if (prec != EH_PREC_PLAIN && prec != EH_PREC_AUTO) return false;
+  if (n == 1 || many_large_tiles(std::is_same<T, double>::value, 2 * m, n) || !operand_fits<T>(ta, ta ? m : 2 * m, ta ? 2 * k : k, 2 * lda) ||
+      !operand_fits<T>(true, n, 2 * k, ldb3))
+    return false;
+  GemmParams<T> p = product_params<T>(false, false, 2 * m, n, 2 * k, ar, A, lda, B3, ldb3, beta, C, 2 * ldc);
+  p.bytesA = (uint32_t)((ta ? (uint64_t)(m - 1) * lda + k : (uint64_t)(k - 1) * lda + m) * 2 * sizeof(T));
+  p.alpha_im = ai;
+  p.conj = conj;
+  *st = launch_balanced<T>(p, kComplexA, ta, false, stream);
+  return true;
+}
+template bool complex_a_product<float>(bool, bool, int64_t, int64_t, int64_t, float, float, const float*, int64_t,
+                                       const float*, int64_t, float, float*, int64_t, int, hipStream_t, eh_status*);
+template bool complex_a_product<double>(bool, bool, int64_t, int64_t, int64_t, double, double, const double*, int64_t,
+                                        const double*, int64_t, double, double*, int64_t, int, hipStream_t,
+                                        eh_status*);
 
 // A product with one output column (n == 1) or row (m == 1) is a
 // matrix-vector product: C^T = op(B)^T op(A)^T turns the row case into the
@@ -611,6 +764,17 @@ static eh_status run_gemm(int opa, int opb, int64_t m, int64_t n, int64_t k, T a
   if (!split_prec && config < 0) {
     eh_status st = plan_config(std::is_same<T, float>::value ? EH_F32 : EH_F64, opa, opb, m, n, k, &config);
     if (st != EH_SUCCESS) return st;
+    if (tune_mode() == EH_TUNE_MLP && !mlp_installed() && operand_fits<T>(ta, m, k, lda) &&
+        operand_fits<T>(!tb, n, k, ldb)) {
+      if (balanced_pays(std::is_same<T, double>::value, m, n, k, config) && balanced_workspace_allowed(stream)) {
+        // the workspace grows to what `config` needs too: a caller may run a
+        // product once before it captures it
+        int t = 0, splits = 1;
+        config_decode(config, &t, &splits);
+        return launch_balanced<T>(product_params<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc), kPlain, ta,
+                                  tb, stream, splits > 1 ? (size_t)splits * m * n * sizeof(T) : 0);
+      }
+    }
   }
   return launch_product<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, split_prec, terms, config, stream);
 }

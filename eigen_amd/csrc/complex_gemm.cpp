@@ -4,10 +4,12 @@
 // Host steps: argument checks with ?gemm_'s rules (blas/level3_impl.h:61-78,
 // complex elements), the quick returns (m == 0 or n == 0; alpha == 0 or
 // k == 0 leaves beta*C), a complex beta applied by a scaling pass (the real
-// product can only apply a real beta), the repack of op(A) with alpha folded
-// in (and of op(B) unless it is B itself), then ONE real product
-// (2m) x n x (2k) through the same planner and kernels as eh_gemm, writing C
-// in place.
+// product can only apply a real beta), the repack of op(B) unless it is B
+// itself, then ONE real product (2m) x n x (2k), writing C in place.  In plain
+// precision the product kernel reads A itself and forms its 2x2 real blocks
+// (times alpha) while it stages them; split precisions, one column,
+// large products and operands past 32-bit addressing repack A and run the planner's real
+// product.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,23 +38,28 @@ eh_status run(int dtype, int opa, int opb, int64_t m, int64_t n, int64_t k, cons
     if (vanishes) return EH_SUCCESS;
     beff = T(1);
   }
-  const bool pack_b = opb != EH_OP_N;
-  StreamTemp t;
-  const size_t a3 = (size_t)4 * m * k, b3 = pack_b ? (size_t)2 * k * n : 0;
-  eh_status st = t.get((a3 + b3) * sizeof(T), s, "complex product temporary");
-  if (st != EH_SUCCESS) return st;
-  T* A3 = static_cast<T*>(t.ptr);
-  hipError_t e = launch_complex_pack_a<T>(A, lda, (int)m, (int)k, opa != EH_OP_N, opa == EH_OP_C, ar, ai, A3, 2 * m, s);
-  if (e != hipSuccess) return hip_fail(e, "complex pack launch");
   const T* B3 = B;
   int64_t ldb3 = 2 * ldb;
-  if (pack_b) {
-    T* P = A3 + a3;
-    e = launch_complex_pack_b<T>(B, ldb, (int)k, (int)n, true, opb == EH_OP_C, P, 2 * k, s);
+  StreamTemp tb;
+  if (opb != EH_OP_N) {
+    eh_status st = tb.get((size_t)2 * k * n * sizeof(T), s, "complex product temporary");
+    if (st != EH_SUCCESS) return st;
+    T* P = static_cast<T*>(tb.ptr);
+    hipError_t e = launch_complex_pack_b<T>(B, ldb, (int)k, (int)n, true, opb == EH_OP_C, P, 2 * k, s);
     if (e != hipSuccess) return hip_fail(e, "complex pack launch");
     B3 = P;
     ldb3 = 2 * k;
   }
+  eh_status st = EH_SUCCESS;
+  if (complex_a_product<T>(opa != EH_OP_N, opa == EH_OP_C, m, n, k, ar, ai, A, lda, B3, ldb3, beff, C, ldc, prec, s,
+                           &st))
+    return st;
+  StreamTemp ta;
+  st = ta.get((size_t)4 * m * k * sizeof(T), s, "complex product temporary");
+  if (st != EH_SUCCESS) return st;
+  T* A3 = static_cast<T*>(ta.ptr);
+  hipError_t e = launch_complex_pack_a<T>(A, lda, (int)m, (int)k, opa != EH_OP_N, opa == EH_OP_C, ar, ai, A3, 2 * m, s);
+  if (e != hipSuccess) return hip_fail(e, "complex pack launch");
   const T one = T(1);
   return gemm_dispatch(dtype, EH_OP_N, EH_OP_N, 2 * m, n, 2 * k, &one, A3, 2 * m, B3, ldb3, &beff, C, 2 * ldc, prec, -1,
                        s);

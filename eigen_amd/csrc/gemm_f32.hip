@@ -37,6 +37,39 @@ hipError_t launch_gemm_mfma(const GemmParams<T>& p, int tile, bool ta, bool tb, 
   }
 }
 
+template <typename T, bool TA, bool TB, int MODE>
+static hipError_t launch_balanced_one(const GemmParams<T>& p, int groups, unsigned* tickets, hipStream_t s) {
+  const BalancedLine<T> line(p, MODE);
+  hipLaunchKernelGGL((gemm_balanced_kernel<T, TA, TB, MODE>), dim3(groups > 0 ? groups : line.lines * line.cols),
+                     dim3(256), 0, s, p, line.units(), groups > 0 ? tickets : nullptr);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_gemm_balanced(const GemmParams<T>& p, int mode, bool ta, bool tb, int groups, unsigned* tickets,
+                                hipStream_t s) {
+  switch (mode * 4 + ta * 2 + tb) {
+    case kPlain * 4: return launch_balanced_one<T, false, false, kPlain>(p, groups, tickets, s);
+    case kPlain * 4 + 1: return launch_balanced_one<T, false, true, kPlain>(p, groups, tickets, s);
+    case kPlain * 4 + 2: return launch_balanced_one<T, true, false, kPlain>(p, groups, tickets, s);
+    case kPlain * 4 + 3: return launch_balanced_one<T, true, true, kPlain>(p, groups, tickets, s);
+    case kComplexA * 4: return launch_balanced_one<T, false, false, kComplexA>(p, groups, tickets, s);
+    case kComplexA * 4 + 2: return launch_balanced_one<T, true, false, kComplexA>(p, groups, tickets, s);
+    case kTriA * 4: return launch_balanced_one<T, false, false, kTriA>(p, groups, tickets, s);
+    case kTriA * 4 + 2: return launch_balanced_one<T, true, false, kTriA>(p, groups, tickets, s);
+    case kTriB * 4: return launch_balanced_one<T, false, false, kTriB>(p, groups, tickets, s);
+    case kTriB * 4 + 1: return launch_balanced_one<T, false, true, kTriB>(p, groups, tickets, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <typename T>
+void balanced_extent(const GemmParams<T>& p, int mode, int64_t* tiles, int64_t* units) {
+  const BalancedLine<T> line(p, mode);
+  *tiles = (int64_t)line.lines * line.cols;
+  *units = line.units();
+}
+
 template <typename T>
 hipError_t launch_splitk_reduce(const GemmParams<T>& p, int splits, hipStream_t s) {
   const int64_t total = (int64_t)p.M * p.N;
@@ -58,6 +91,8 @@ hipError_t launch_scale_c(T* C, int M, int N, int64_t ldc, T beta, hipStream_t s
 }
 
 template hipError_t launch_gemm_mfma<float>(const GemmParams<float>&, int, bool, bool, int, hipStream_t);
+template hipError_t launch_gemm_balanced<float>(const GemmParams<float>&, int, bool, bool, int, unsigned*, hipStream_t);
+template void balanced_extent<float>(const GemmParams<float>&, int, int64_t*, int64_t*);
 template hipError_t launch_splitk_reduce<float>(const GemmParams<float>&, int, hipStream_t);
 template hipError_t launch_scale_c<float>(float*, int, int, int64_t, float, hipStream_t, int);
 

@@ -33,19 +33,30 @@ inline int64_t grid_tiles(const GemmParams<T>& p) {
   return tri_compact<BM, BN>(p) ? ntm * (ntm + 1) / 2 : ntm * ntn;
 }
 
-// LDS bytes of one tile body: two stages of (BM + BN) rows of 128 bytes.
+// LDS bytes of one tile_product: two stages of (BM + BN) rows of 128 bytes.
 template <int BM, int BN>
 constexpr int tile_smem_bytes() {
   return 2 * (BM + BN) * 128;
 }
 
-// One BM x BN tile of C at (m0, n0) over k in [kbeg, kend): the whole body of
-// a product workgroup (gemm_mfma_kernel below).  z / partial: split-K
-// slice and whether the result goes to the partial buffer p.W.  smem holds
-// tile_smem_bytes<BM, BN>(); the caller synchronises before reusing it.
-template <typename T, int BM, int BN, int WGM, int WGN, bool TA, bool TB, int RS>
-__device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int kbeg, int kend, int z,
-                                          bool partial, unsigned char* __restrict__ smem) {
+// One BM x BN tile of op(A)*op(B) at (m0, n0) over k in [kbeg, kend): the body
+// of a product workgroup.  At the end epi(acc) takes the wave's accumulators.
+// smem holds tile_smem_bytes<BM, BN>(); the caller synchronises before reusing
+// it.
+// MODE: operand forms read in place of a repacked copy.
+//   kComplexA      A holds interleaved (re, im) pairs (lda in pairs): each
+//                  pair is staged as the 2x2 real block of alpha * op(A)
+//                  (conjugated when p.conj), so M and K are twice op(A)'s.
+//   kTriA, kTriB   op(A) (op(B)) is triangular, lower or upper by p.lower:
+//                  elements off the triangle are staged as zeros whatever the
+//                  memory holds, the diagonal as ones when p.unit.
+// FOLD: every 128 of k the accumulators are added to a second set and start
+// again from zero, so that a sum over one long run of k rounds no worse than
+// one cut into splits or blocks (FP32 TRMM 1500 x 1100: relative error 2.1e-7
+// against 3.6e-7 in one chain and 2.5e-7 over 256-row leaves).
+template <typename T, int BM, int BN, int WGM, int WGN, bool TA, bool TB, int RS, int MODE, bool FOLD, typename Epi>
+__device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int kbeg, int kend,
+                                          unsigned char* __restrict__ smem, Epi epi) {
   using F = Mfma<T>;
   constexpr int NT = 64 * WGM * WGN;
   constexpr int ROWB = 128;                // bytes of k per LDS row
@@ -56,7 +67,9 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
   constexpr int RM = WTM / F::MI, RN = WTN / F::NI;
   constexpr int KPL = BK / F::KG;          // k values one lane feeds per slice
   constexpr int CPL = KPL / EPC;           // chunks one lane reads per row
-  constexpr int A_CH = BM * CH / NT, B_CH = BN * CH / NT;
+  // chunks a thread loads per slice (a complex chunk makes two LDS chunks)
+  constexpr int A_CH = BM * CH / NT / (MODE == kComplexA ? 2 : 1), B_CH = BN * CH / NT;
+  constexpr int AR = MODE == kComplexA ? BM / 2 : BM;  // rows of op(A) in the tile
   static_assert(RM >= 1 && RN >= 1, "wave tile smaller than one MFMA block");
   static_assert(BM * CH % NT == 0 && BN * CH % NT == 0, "tile not divisible by threads");
   static_assert(CPL * EPC == KPL, "lane k range must be whole chunks");
@@ -86,9 +99,15 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
     const int q = tid + NT * j;
     if constexpr (TA) {  // op(A)(i,k) = A[k + i*lda]: k contiguous
       const int r = q / CH, c = q % CH;
-      voA[j] = (uint32_t)(((uint64_t)(m0 + r) * p.lda + c * EPC) * SZ);
+      if constexpr (MODE == kComplexA)
+        voA[j] = (uint32_t)(((uint64_t)(m0 / 2 + r) * p.lda * 2 + c * EPC) * SZ);
+      else
+        voA[j] = (uint32_t)(((uint64_t)(m0 + r) * p.lda + c * EPC) * SZ);
     } else {  // op(A)(i,k) = A[i + k*lda]: rows contiguous
-      voA[j] = (uint32_t)((m0 + q % BM) * SZ);
+      if constexpr (MODE == kComplexA)  // with the chunk's first k: a wave's lanes may hold two chunks
+        voA[j] = (uint32_t)((m0 + 2 * (q % AR) + (uint64_t)(q / AR * EPC) * p.lda) * SZ);
+      else
+        voA[j] = (uint32_t)((m0 + q % AR) * SZ);
     }
   }
 #pragma unroll
@@ -118,6 +137,18 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
       t[e] = buf_load(rs, vo, (uint32_t)((uint64_t)(k0 + cu * EPC + e) * ld * SZ), (T*)nullptr);
     return *reinterpret_cast<u32x4*>(t);
   };
+  // the same for complex pairs: the pair of one k (FP64) or of two (FP32)
+  auto load_pairs = [&](uint32_t vo, int k0) -> u32x4 {
+    const uint32_t so = (uint32_t)((uint64_t)k0 * p.lda * SZ);
+    if constexpr (SZ == 8) {
+      return buf_load16(rA, vo, so);
+    } else {
+      typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+      const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(rA, (int)vo, (int)so, 0);
+      const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(rA, (int)(vo + (uint32_t)p.lda * 8), (int)so, 0);
+      return u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+  };
   // slice s (clamped to the last one: a prefetch past the end re-reads it)
   auto load = [&](Stage& st, int s) {
     const int k0 = kbeg + min(s, nkt - 1) * BK;
@@ -126,8 +157,10 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
       const int q = tid + NT * j;
       if constexpr (TA)
         st.a[j] = buf_load16(rA, voA[j], (uint32_t)k0 * SZ);
+      else if constexpr (MODE == kComplexA)
+        st.a[j] = load_pairs(voA[j], k0);
       else
-        st.a[j] = load_mncont(rA, voA[j], k0, __builtin_amdgcn_readfirstlane(q / BM), p.lda);
+        st.a[j] = load_mncont(rA, voA[j], k0, __builtin_amdgcn_readfirstlane(q / AR), p.lda);
     }
 #pragma unroll
     for (int j = 0; j < B_CH; ++j) {
@@ -145,6 +178,17 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
 #pragma unroll
     for (int e = 0; e < EPC; ++e) t[e] = (k0 + c * EPC + e < kend) ? t[e] : T(0);
   };
+  // chunk of line i (row of op(A), column of op(B)) at k..: elements off the
+  // triangle become zeros; keep k <= i or k >= i
+  auto mask_tri = [&](u32x4& v, int i, int k, bool keep_below) {
+    T* t = reinterpret_cast<T*>(&v);
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) {
+      const int d = keep_below ? i - k - e : k + e - i;
+      t[e] = d < 0 ? T(0) : t[e];
+      t[e] = (d == 0) & (p.unit != 0) ? T(1) : t[e];
+    }
+  };
   // ---- registers -> LDS buffer -------------------------------------------
   auto store = [&](Stage& st, int s, int buf) {
     const int k0 = kbeg + min(s, nkt - 1) * BK;
@@ -153,15 +197,35 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
 #pragma unroll
     for (int j = 0; j < A_CH; ++j) {
       const int q = tid + NT * j;
-      const int r = TA ? q / CH : q % BM, c = TA ? q % CH : q / BM;
+      const int r = TA ? q / CH : q % AR, c = TA ? q % CH : q / AR;
       if constexpr (TA) mask_kcont(st.a[j], k0, c);
-      *reinterpret_cast<u32x4*>(As + r * ROWB + swz8(r, c) * 16) = st.a[j];
+      if constexpr (MODE == kTriA) mask_tri(st.a[j], m0 + r, k0 + c * EPC, p.lower);
+      if constexpr (MODE == kComplexA) {
+        // alpha * op(A)(i, k) = (x, y): row 2i holds (x, -y), row 2i + 1 (y, x)
+        const T* t = reinterpret_cast<const T*>(&st.a[j]);
+        u32x4 lo, hi;
+        T *rl = reinterpret_cast<T*>(&lo), *rh = reinterpret_cast<T*>(&hi);
+#pragma unroll
+        for (int e = 0; e < EPC; e += 2) {
+          const T im = p.conj ? -t[e + 1] : t[e + 1];
+          const T x = p.alpha * t[e] - p.alpha_im * im, y = p.alpha * im + p.alpha_im * t[e];
+          rl[e] = x;
+          rl[e + 1] = -y;
+          rh[e] = y;
+          rh[e + 1] = x;
+        }
+        *reinterpret_cast<u32x4*>(As + (2 * r) * ROWB + swz8(2 * r, c) * 16) = lo;
+        *reinterpret_cast<u32x4*>(As + (2 * r + 1) * ROWB + swz8(2 * r + 1, c) * 16) = hi;
+      } else {
+        *reinterpret_cast<u32x4*>(As + r * ROWB + swz8(r, c) * 16) = st.a[j];
+      }
     }
 #pragma unroll
     for (int j = 0; j < B_CH; ++j) {
       const int q = tid + NT * j;
       const int r = TB ? q % BN : q / CH, c = TB ? q / BN : q % CH;
       if constexpr (!TB) mask_kcont(st.b[j], k0, c);
+      if constexpr (MODE == kTriB) mask_tri(st.b[j], n0 + r, k0 + c * EPC, !p.lower);
       *reinterpret_cast<u32x4*>(Bs + r * ROWB + swz8(r, c) * 16) = st.b[j];
     }
   };
@@ -210,6 +274,20 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
     }
   };
 
+  typename F::acc_t total[FOLD ? RM : 1][FOLD ? RN : 1] = {};
+  auto fold = [&]() {
+    if constexpr (FOLD) {
+#pragma unroll
+      for (int i = 0; i < RM; ++i)
+#pragma unroll
+        for (int j = 0; j < RN; ++j) {
+          total[i][j] += acc[i][j];
+          acc[i][j] = typename F::acc_t{};
+        }
+    }
+  };
+  constexpr int FS = 128 / BK;  // slices between folds
+
   if (nkt > 0) {
     if constexpr (RS == 2) {
       // Two register stages: the loads of slice s + 2 are issued while slice
@@ -232,6 +310,7 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
         store(r0, kt + 2, 0);
         __syncthreads();
         load(r0, kt + 4);
+        if (FOLD && kt % FS == FS - 2) fold();
       }
       if (kt < nkt) compute(0);  // odd slice count: the last slice is in buffer 0
     } else {
@@ -248,11 +327,28 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
     }
   }
 
-  // ---- epilogue -------------------------------------------------------------
+  if constexpr (FOLD) {
+    static_assert(RS == 2, "folding runs in the two-stage loop");
+    fold();
+    epi(total);
+  } else {
+    epi(acc);
+  }
+}
+
+// The store of a tile: C = alpha*acc + beta*C, or (partial) acc to split z of
+// the partial buffer p.W.
+template <typename T, int BM, int BN, int WGM, int WGN, typename Acc>
+__device__ __forceinline__ void tile_store(const GemmParams<T>& p, T alpha, int m0, int n0, int z, bool partial,
+                                           const Acc& acc) {
+  using F = Mfma<T>;
+  constexpr int WTM = BM / WGM, WTN = BN / WGN;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int wm = wid % WGM, wn = wid / WGM;
 #pragma unroll
-  for (int i = 0; i < RM; ++i)
+  for (int i = 0; i < WTM / F::MI; ++i)
 #pragma unroll
-    for (int j = 0; j < RN; ++j) {
+    for (int j = 0; j < WTN / F::NI; ++j) {
       const int col = n0 + wn * WTN + j * F::NI + F::col(lane);
       if (col >= p.N) continue;
 #pragma unroll
@@ -264,7 +360,7 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
         } else {
           T* dst = p.C + row + (int64_t)col * p.ldc;
           T v = acc[i][j][r];
-          *dst = (p.beta == T(0)) ? p.alpha * v : fma_t(p.alpha, v, p.beta * *dst);
+          *dst = (p.beta == T(0)) ? alpha * v : fma_t(alpha, v, p.beta * *dst);
         }
       }
     }
@@ -290,7 +386,186 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_mfma_kernel(GemmParams<T>
   const int z = blockIdx.y;
   const int kbeg = z * p.k_per_split;
   const int kend = min(p.K, kbeg + p.k_per_split);
-  gemm_tile<T, BM, BN, WGM, WGN, TA, TB, RS>(p, m0, n0, kbeg, kend, z, gridDim.y > 1, smem);
+  gemm_tile<T, BM, BN, WGM, WGN, TA, TB, RS, kPlain, false>(
+      p, m0, n0, kbeg, kend, smem,
+      [&](const auto& acc) { tile_store<T, BM, BN, WGM, WGN>(p, p.alpha, m0, n0, z, gridDim.y > 1, acc); });
+}
+
+// ---------------------------------------------------------------------------
+// Balanced product: the tiles' k slices, one tile's after another's, are one
+// line of units, cut into gridDim.x equal runs (all resident at once), so
+// neither a tile count that is no multiple of what the chip holds nor tiles
+// of unequal depth (a triangular operand) leave anything idle.  Tiles are
+// 64x64 with four waves, three workgroups per CU: 128x128 tiles, two per CU,
+// lose more to the larger cut tiles than they gain (FP64 1000x777x1203 86
+// against 50 us, 2048x700x3000 190 against 159, FP32 1645x1384x2732 132 against
+// 123); so do wave groups that share a tile's k slices (58, 178 us for four).
+//
+// A tile that lies inside one run is stored at once.  Of a tile cut between
+// runs every workgroup writes its part to a slot (the first segment of run g
+// to slot 2g, its last to 2g + 1) and takes a ticket; whoever takes the last
+// one adds the parts, in run order, so the result does not depend on who that
+// is, and clears the ticket.  Nobody waits for anybody.
+// Without tickets every workgroup takes one whole tile.
+// ---------------------------------------------------------------------------
+// The parts travel between workgroups on different XCDs, whose L2s are not
+// coherent: their stores and loads carry the device scope bit (sc1), which
+// writes and reads past the L2, so no cache has to be written back or
+// invalidated (a __threadfence per wave did that: FP64 1000x777x1203 took 126
+// us instead of 59).
+__device__ inline void slot_store(__amdgpu_buffer_rsrc_t r, uint32_t off, u32x4 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, 16);
+}
+__device__ inline u32x4 slot_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 16);
+}
+
+// The line of units of a product, on the host and in the kernel: lines of
+// `cols` tiles, all tiles of line r over the k slices [begin(r), begin(r) +
+// slices(r)*bk).  A dense product is one line of all tiles; a triangular
+// operand gives one line per tile row of op(A) (tile column of op(B)), each of
+// its tiles lengthened by kTileCost units that stand for the tile's first loads
+// and its store (FP32 TRMM 1500 x 1100: 80, 49, 55 us with 0, 4, 10; FP64 3000 x
+// 2900: 700, 575, 596).
+constexpr int kTileCost = 4;
+template <typename T>
+struct BalancedLine {
+  int lines, cols, K, bt, bk, mode;
+  bool from0;  // triangular: k from 0 up to the tile's end, or from the tile's start up to K
+  __host__ __device__ BalancedLine(const GemmParams<T>& p, int m) : mode(m) {
+    constexpr int b = kBalancedTile;
+    const int ntm = (p.M + b - 1) / b, ntn = (p.N + b - 1) / b;
+    lines = m == kTriA ? ntm : m == kTriB ? ntn : 1;
+    cols = m == kTriA ? ntn : m == kTriB ? ntm : ntm * ntn;
+    K = p.K;
+    bt = b;
+    bk = 128 / (int)sizeof(T);
+    from0 = (m == kTriA) == (p.lower != 0);
+  }
+  __host__ __device__ int begin(int r) const { return mode < kTriA || from0 ? 0 : r * bt; }
+  __host__ __device__ int end(int r) const { return mode < kTriA || !from0 || (r + 1) * bt > K ? K : (r + 1) * bt; }
+  __host__ __device__ int slices(int r) const { return (end(r) - begin(r) + bk - 1) / bk; }
+  __host__ __device__ int span(int r) const { return slices(r) + (mode < kTriA ? 0 : kTileCost); }
+  __host__ __device__ int64_t units() const {
+    int64_t u = 0;
+    for (int r = 0; r < lines; ++r) u += (int64_t)cols * span(r);
+    return u;
+  }
+};
+
+template <typename T, bool TA, bool TB, int MODE>
+__global__ void __launch_bounds__(256, 3) gemm_balanced_kernel(GemmParams<T> p, int64_t units, unsigned* tickets) {
+  using F = Mfma<T>;
+  constexpr int BM = kBalancedTile, BN = kBalancedTile;
+  constexpr int RM = BM / 2 / F::MI, RN = BN / 2 / F::NI;
+  constexpr int BK = 128 / sizeof(T);
+  constexpr int NT = 256;
+  constexpr int VPB = F::ACC * sizeof(T) / 16;  // 16-byte vectors of one lane per MFMA block
+  constexpr int NB = RM * RN;
+  constexpr int CB = NB * VPB > 8 ? 8 / VPB : NB;  // blocks a thread adds up at a time (32 registers of parts)
+  constexpr int SLOT = BM * BN * sizeof(T);     // bytes of a slot
+  __shared__ __attribute__((aligned(16))) unsigned char smem[tile_smem_bytes<BM, BN>()];
+  __shared__ int flag;
+  const BalancedLine<T> line(p, MODE);
+  const int64_t G = gridDim.x;
+  const int64_t g = xcd_remap(blockIdx.x, gridDim.x);
+  int r = 0;         // line of the current tile
+  int64_t base = 0;  // first unit of that line
+  int span = line.span(0);
+  int64_t u0, u1;
+  if (tickets) {
+    u0 = units * g / G;
+    u1 = units * (g + 1) / G;
+    while (u0 >= base + (int64_t)line.cols * span) {
+      base += (int64_t)line.cols * span;
+      span = line.span(++r);
+    }
+  } else {
+    r = (int)(g / line.cols);
+    span = line.span(r);
+    u0 = (g % line.cols) * span;
+    u1 = u0 + span;
+  }
+  auto slot_rsrc = [&](int64_t i) {
+    return make_rsrc(reinterpret_cast<unsigned char*>(p.W) + i * SLOT, (uint32_t)SLOT);
+  };
+  for (int64_t u = u0, end; u < u1; u = end) {
+    if (u == base + (int64_t)line.cols * span) {
+      base = u;
+      span = line.span(++r);
+    }
+    const int c = (int)((u - base) / span), S = line.slices(r);
+    const int64_t first = base + (int64_t)c * span;
+    end = min(u1, first + span);
+    const int s0 = (int)(u - first), s1 = min((int)(end - first), S);
+    if (s0 >= S) continue;
+    int tm, tn;
+    if constexpr (MODE == kTriA) {
+      tm = r;
+      tn = c;
+    } else if constexpr (MODE == kTriB) {
+      tm = c;
+      tn = r;
+    } else {
+      tile_coords(c, (p.M + BM - 1) / BM, (p.N + BN - 1) / BN, 8, tm, tn);
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int kb = line.begin(r);
+    auto finish = [&](auto& acc) {
+      bool store = true;
+      if (s0 != 0 || s1 != S) {
+        unsigned* ticket = tickets + (int64_t)r * line.cols + c;
+        // runs g0..g1 meet this tile: run h owns unit x for h = floor(((x + 1)G - 1) / units)
+        const int64_t g0 = ((first + 1) * G - 1) / units, g1 = ((first + S) * G - 1) / units;
+        const unsigned others = (unsigned)(g1 - g0);
+        const __amdgpu_buffer_rsrc_t mine = slot_rsrc(2 * g + (u == u0 ? 0 : 1));
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const u32x4* a = reinterpret_cast<const u32x4*>(&acc[b / RN][b % RN]);
+#pragma unroll
+          for (int v = 0; v < VPB; ++v) slot_store(mine, (uint32_t)(((b * VPB + v) * NT + threadIdx.x) * 16), a[v]);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part has reached memory
+        __syncthreads();
+        if (threadIdx.x == 0) {
+          flag = atomicAdd(ticket, 1u) == others;
+          if (flag) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        store = flag;
+        if (store) {
+          // CB blocks at a time, two parts in flight
+#pragma unroll
+          for (int b0 = 0; b0 < NB; b0 += CB) {
+            typename F::acc_t sum[CB] = {};
+            for (int64_t h = g0; h <= g1; h += 2) {
+              u32x4 w[2][CB * VPB];
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                const int64_t hh = h + i <= g1 ? h + i : g1;
+                const __amdgpu_buffer_rsrc_t part = slot_rsrc(2 * hh + (units * hh / G >= first ? 0 : 1));
+#pragma unroll
+                for (int v = 0; v < CB * VPB; ++v)
+                  w[i][v] = slot_load(part, (uint32_t)(((b0 * VPB + v) * NT + threadIdx.x) * 16));
+              }
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                if (h + i > g1) break;
+#pragma unroll
+                for (int b = 0; b < CB; ++b) sum[b] += *reinterpret_cast<const typename F::acc_t*>(&w[i][b * VPB]);
+              }
+            }
+#pragma unroll
+            for (int b = 0; b < CB; ++b) acc[(b0 + b) / RN][(b0 + b) % RN] = sum[b];
+          }
+        }
+      }
+      if (store) tile_store<T, BM, BN, 2, 2>(p, MODE == kComplexA ? T(1) : p.alpha, m0, n0, 0, false, acc);
+    };
+    gemm_tile<T, BM, BN, 2, 2, TA, TB, 2, MODE, true>(p, m0, n0, kb + s0 * BK, min(line.end(r), kb + s1 * BK), smem,
+                                                      finish);
+    __syncthreads();  // smem and flag are free again
+  }
 }
 
 // Deterministic split-K reduction: C = alpha * sum_z W[z] + beta*C.

@@ -38,14 +38,18 @@ int plan_packed(int kind, int opa, int opb, int64_t m, int64_t n, int64_t k);
 eh_status packed_product(int kind, int opa, int opb, int64_t m, int64_t n, int64_t k, const void* A, const void* B,
                          void* C, int config, hipStream_t s);
 
+constexpr size_t kTicketBytes = 4 * 8192;  // one per tile of a balanced product
+
 // Per-stream device workspace (capi.cpp).  A lease holds the stream's
 // workspace lock and a reference to its buffer: hold it until every launch
 // of the call that uses the buffer is queued, so that another thread's call
 // on the same stream can neither interleave its launches with ours (both
 // would use the one buffer) nor free the buffer under us.
 struct Workspace {
+  void* base = nullptr;  // kTicketBytes of tickets, then the buffer
   void* ptr = nullptr;
   size_t bytes = 0;
+  bool tickets_clear = false;
   Workspace() = default;
   Workspace(const Workspace&) = delete;
   Workspace& operator=(const Workspace&) = delete;
@@ -127,6 +131,22 @@ template <typename R>
 eh_status complex_product(int opa, int opb, int64_t m, int64_t n, int64_t k, cplx<R> alpha, const cplx<R>* A,
                           int64_t lda, const cplx<R>* B, int64_t ldb, cplx<R> beta, cplx<R>* C, int64_t ldc,
                           hipStream_t s);
+// C = alpha*E*X (left) or alpha*X*E, E the order x order triangle at E (tri_t:
+// transposed, so E(i, k) = E[k + i*lde]; lower: of the operator; unit
+// diagonal), X and C with `other` columns (left) or rows; one launch that
+// multiplies only the triangle.  C must not overlap X.  Returns false
+// (nothing done) when an operand is past 32-bit addressing.
+template <typename T>
+bool tri_product(bool left, bool tri_t, bool lower, bool unit, int64_t order, int64_t other, T alpha, const T* E,
+                 int64_t lde, const T* X, int64_t ldx, T* C, int64_t ldc, hipStream_t stream, eh_status* st);
+// Complex product with A read in place (interleaved pairs, lda and ldc in
+// pairs) and B3 the real 2k x n form of op(B); beta real.  Returns false
+// (nothing done) for split precisions, one column, products large enough for
+// 128x128 tiles, and operands past 32-bit addressing.
+template <typename T>
+bool complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,
+                       const T* B3, int64_t ldb3, T beta, T* C, int64_t ldc, int prec, hipStream_t stream,
+                       eh_status* st);
 eh_status gemm_dispatch(int dtype, int opa, int opb, int64_t m, int64_t n, int64_t k, const void* alpha,
                         const void* A, int64_t lda, const void* B, int64_t ldb, const void* beta, void* C,
                         int64_t ldc, int prec, int config, void* stream);

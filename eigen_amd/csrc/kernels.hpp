@@ -28,11 +28,28 @@ struct GemmParams {
   // Triangle of C the product updates: 0 all of it, 1 the lower (row >= col),
   // 2 the upper (row <= col); the rest of C is neither read nor written.
   int tri;
+  // Balanced product with an operand form (gemm_mfma.hpp): imaginary part of
+  // alpha and conjugation of a complex A; triangle of a triangular operand.
+  T alpha_im = T(0);
+  int conj = 0, lower = 0, unit = 0;
 };
 
 // Plain MFMA product: tile 0..5 = 64x64, 64x128, 128x64, 128x128, 128x256, 256x128.
 template <typename T>
 hipError_t launch_gemm_mfma(const GemmParams<T>& p, int tile, bool ta, bool tb, int splits, hipStream_t s);
+// Operand forms of the balanced product.
+enum { kPlain = 0, kComplexA = 1, kTriA = 2, kTriB = 3 };
+constexpr int kBalancedTile = 64;
+// Balanced product (gemm_balanced_kernel).  kComplexA takes op(B) = B; kTriA /
+// kTriB the other operand not transposed.  `groups` workgroups share the k
+// slices of all tiles; p.W holds two tiles per workgroup, tickets one zero word
+// per tile.  groups = 0: one workgroup per tile, no p.W or tickets.
+template <typename T>
+hipError_t launch_gemm_balanced(const GemmParams<T>& p, int mode, bool ta, bool tb, int groups, unsigned* tickets,
+                                hipStream_t s);
+// Tiles of that product, and the length of their line of k slices.
+template <typename T>
+void balanced_extent(const GemmParams<T>& p, int mode, int64_t* tiles, int64_t* units);
 template <typename T>
 hipError_t launch_splitk_reduce(const GemmParams<T>& p, int splits, hipStream_t s);
 template <typename T>

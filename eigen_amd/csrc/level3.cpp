@@ -9,8 +9,8 @@
 //   SYMM           the mirrored dense matrix (one HBM pass), then one product;
 //   TRMM, TRSM     recursive 2x2 blocking of the triangle: at each level the
 //                  off-diagonal block is a plain product on the rest of B;
-//                  the leaves are products too (TRMM: the dense diagonal
-//                  block; complex TRSM: the inverse of the diagonal block,
+//                  the leaves are products too (TRMM: the triangle itself,
+//                  for complex types the dense diagonal block; complex TRSM: the inverse of the diagonal block,
 //                  all of them computed by one launch).  Real TRSM runs
 //                  panels of rows instead (trsm_panels).
 // Arguments are checked with the reference's rules (blas/level3_impl.h); the
@@ -207,15 +207,37 @@ eh_status trsm_right(const Tri<T>& E, int64_t d, int64_t sz, T* B, int64_t ldb, 
 }
 
 // ---- TRMM --------------------------------------------------------------------
+// Real types: ranges up to kTrmmLeafReal multiply a copy of their part of B
+// by the triangle itself in one launch (tri_product).  FP32 1500 x 1100 from
+// the right: 51 us, against 180 through 256-row dense leaves (17 launches);
+// FP64 8192 x 8192: 9.4 against 9.9 ms.
+// Complex types, and triangles past 32-bit addressing, expand dense leaves.
 constexpr int64_t kTrmmLeaf = 256;
+constexpr int64_t kTrmmLeafReal = 2048;
+constexpr int64_t kTrmmMaxLd = 1 << 17;
 
 // Workspace of the TRMM leaves: the dense diagonal block and a copy of the
 // part of B it multiplies.
 template <typename T>
 struct TrmmWork {
-  T* dense;  // kTrmmLeaf x kTrmmLeaf
+  T* dense;  // leaf x leaf; null: the leaves read the triangle in place
   T* copy;   // leaf rows x n (left) or m x leaf columns (right)
+  int64_t leaf;
 };
+
+// Leaf with the triangle read in place: copy the sz rows (left) or columns
+// of B, then one triangular product.
+template <typename T>
+eh_status trmm_leaf(const Tri<T>& E, bool left, int64_t d, int64_t sz, T* B, int64_t ldb, int64_t other, T alpha,
+                    const TrmmWork<T>& w, hipStream_t s) {
+  const int64_t rows = left ? sz : other, cols = left ? other : sz;
+  hipError_t e = launch_copy_block<T>(B, ldb, (int)rows, (int)cols, w.copy, s);
+  if (e != hipSuccess) return hip_fail(e, "trmm block copy launch");
+  eh_status st = EH_SUCCESS;
+  if (!tri_product<T>(left, E.ta, E.lower, E.unit, sz, other, alpha, E.diag(d), E.lda, w.copy, rows, B, ldb, s, &st))
+    return fail(EH_ERR_UNSUPPORTED, "triangular product past 32-bit addressing");
+  return st;
+}
 
 template <typename T>
 eh_status dense_diag(const Tri<T>& E, int64_t d, int64_t sz, T* D, hipStream_t s) {
@@ -227,14 +249,16 @@ eh_status dense_diag(const Tri<T>& E, int64_t d, int64_t sz, T* D, hipStream_t s
 template <typename T>
 eh_status trmm_left(const Tri<T>& E, int64_t d, int64_t sz, T* B, int64_t ldb, int64_t n, T alpha,
                     const TrmmWork<T>& w, hipStream_t s) {
-  if (sz <= kTrmmLeaf) {
+  if (sz <= w.leaf) {
+    if constexpr (!IsCplx<T>::value)
+      if (!w.dense) return trmm_leaf(E, true, d, sz, B, ldb, n, alpha, w, s);
     EH_TRY(dense_diag(E, d, sz, w.dense, s));
     hipError_t e = hipMemcpy2DAsync(w.copy, sz * sizeof(T), B, ldb * sizeof(T), sz * sizeof(T), n,
                                     hipMemcpyDeviceToDevice, s);
     if (e != hipSuccess) return hip_fail(e, "trmm block copy");
     return prod(E.op(), EH_OP_N, sz, n, sz, alpha, w.dense, sz, w.copy, sz, T(0), B, ldb, s);
   }
-  const int64_t h = half(sz, kTrmmLeaf);
+  const int64_t h = half(sz, w.leaf);
   T* B1 = B;
   T* B2 = B + h;
   if (E.lower) {  // B2 = alpha*(E22*B2 + E21*B1) before B1 changes
@@ -254,14 +278,16 @@ eh_status trmm_left(const Tri<T>& E, int64_t d, int64_t sz, T* B, int64_t ldb, i
 template <typename T>
 eh_status trmm_right(const Tri<T>& E, int64_t d, int64_t sz, T* B, int64_t ldb, int64_t m, T alpha,
                      const TrmmWork<T>& w, hipStream_t s) {
-  if (sz <= kTrmmLeaf) {
+  if (sz <= w.leaf) {
+    if constexpr (!IsCplx<T>::value)
+      if (!w.dense) return trmm_leaf(E, false, d, sz, B, ldb, m, alpha, w, s);
     EH_TRY(dense_diag(E, d, sz, w.dense, s));
     hipError_t e = hipMemcpy2DAsync(w.copy, m * sizeof(T), B, ldb * sizeof(T), m * sizeof(T), sz,
                                     hipMemcpyDeviceToDevice, s);
     if (e != hipSuccess) return hip_fail(e, "trmm block copy");
     return prod(EH_OP_N, E.op(), m, sz, sz, alpha, w.copy, m, w.dense, sz, T(0), B, ldb, s);
   }
-  const int64_t h = half(sz, kTrmmLeaf);
+  const int64_t h = half(sz, w.leaf);
   T* B1 = B;
   T* B2 = B + h * ldb;
   if (E.lower) {  // B1 = alpha*(B1*E11 + B2*E21) before B2 changes
@@ -343,11 +369,15 @@ eh_status trmm_t(int side, int uplo, int transa, int diag, int64_t m, int64_t n,
   const bool ta = transa != EH_OP_N;
   const Tri<T> E{A, lda, ta, (uplo == EH_LOWER) != ta, diag == EH_UNIT, transa == EH_OP_C};
   const int64_t ka = side == EH_LEFT ? m : n;
-  const int64_t leaf = std::min(ka, kTrmmLeaf);
-  const int64_t copy = side == EH_LEFT ? leaf * n : m * leaf;
+  const int64_t other = side == EH_LEFT ? n : m;
+  // in place: 32-bit offsets over a leaf of the triangle and its copy of B
+  const bool in_place = !IsCplx<T>::value && lda <= kTrmmMaxLd && other <= kTrmmMaxLd;
+  const int64_t leaf = std::min(ka, in_place ? kTrmmLeafReal : kTrmmLeaf);
+  const int64_t dense = in_place ? 0 : leaf * leaf;
   StreamTemp t;
-  EH_TRY(t.get((size_t)(leaf * leaf + copy) * sizeof(T), s, "level-3 temporary"));
-  const TrmmWork<T> w{static_cast<T*>(t.ptr), static_cast<T*>(t.ptr) + leaf * leaf};
+  EH_TRY(t.get((size_t)(dense + leaf * other) * sizeof(T), s, "level-3 temporary"));
+  T* base = static_cast<T*>(t.ptr);
+  const TrmmWork<T> w{in_place ? nullptr : base, base + dense, leaf};
   return side == EH_LEFT ? trmm_left<T>(E, 0, m, B, ldb, n, alpha, w, s)
                          : trmm_right<T>(E, 0, n, B, ldb, m, alpha, w, s);
 }

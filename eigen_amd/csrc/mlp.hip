@@ -227,6 +227,12 @@ bool mlp_has_default() { return false; }
 static bool g_planner_is_default = false;
 #endif
 
+// Whether the planner runs a network its caller set.
+bool mlp_installed() {
+  std::lock_guard<std::mutex> lk(g_mlp_mutex);
+  return !g_planner_is_default;
+}
+
 // Measured best configuration of a shape that was tuned together with the
 // compiled-in network (exact match), or -1.
 static int tuned_shape_plan(int dtype, int opa, int opb, int64_t m, int64_t n, int64_t k) {
