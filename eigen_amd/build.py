@@ -25,14 +25,15 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 HIPFLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
-LIB_SOURCES = ["gemm_f32.hip", "gemm_f64.hip", "gemm_split.hip", "gemv.hip", "level3_kernels.hip", "fill.hip", "grouped.hip",
-               "mlp.hip", "complex_kernels.hip", "noalloc.hip", "level3.cpp", "complex_gemm.cpp",
+LIB_SOURCES = ["gemm_f32.hip", "gemm_f64.hip", "gemm_small.hip", "gemm_split.hip", "gemv.hip", "level3_kernels.hip",
+               "fill.hip", "grouped.hip", "mlp.hip", "complex_kernels.hip", "noalloc.hip", "level3.cpp", "complex_gemm.cpp",
                "capi.cpp", "planner.cpp", "tuner.cpp"]
 BLAS_SOURCES = ["blas.cpp"]
 # Per-file code generation choices.  The FP64 kernels keep their
 # accumulators in the VGPR form of the MFMA: with AGPR accumulators the
 # 128x128 tile copied every accumulator through VGPRs on each k slice.
 FILE_FLAGS = {"gemm_f64.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "gemm_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               # the grouped kernel's accumulators in VGPRs: 112 registers, four waves per SIMD
               "grouped.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               # the solve kernels' small accumulators too (16 copies per slab otherwise)

@@ -37,6 +37,10 @@ struct GemmParams {
 // Plain MFMA product: tile 0..5 = 64x64, 64x128, 128x64, 128x128, 128x256, 256x128.
 template <typename T>
 hipError_t launch_gemm_mfma(const GemmParams<T>& p, int tile, bool ta, bool tb, int splits, hipStream_t s);
+// Plain product of small matrices (gemm_small.hip); operands below 2 GB.
+constexpr int kSmallTile = 32;
+template <typename T>
+hipError_t launch_gemm_small(const GemmParams<T>& p, bool ta, bool tb, hipStream_t s);
 // Operand forms of the balanced product.
 enum { kPlain = 0, kComplexA = 1, kTriA = 2, kTriB = 3 };
 constexpr int kBalancedTile = 64;
