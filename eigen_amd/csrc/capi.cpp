@@ -684,6 +684,17 @@ template bool complex_a_product<double>(bool, bool, int64_t, int64_t, int64_t, d
                                         const double*, int64_t, double, double*, int64_t, int, hipStream_t,
                                         eh_status*);
 
+// Tickets for a split matrix-vector product, or nullptr (the sums are the same
+// bits either way): in a captured call and in the fixed scratch, and for more
+// row blocks than there are tickets.
+static unsigned* gemv_tickets(const GemvPlan& g, hipStream_t stream, WorkspaceLease& lease) {
+  unsigned* tickets = nullptr;
+  if (g.splits == 1 || !lease.buf || g.blocks > (int)(kTicketBytes / 4) || !balanced_workspace_allowed(stream) ||
+      workspace_tickets(stream, lease, &tickets) != EH_SUCCESS)
+    return nullptr;
+  return tickets;
+}
+
 // A product with one output column (n == 1) or row (m == 1) is a
 // matrix-vector product: C^T = op(B)^T op(A)^T turns the row case into the
 // column case.  Returns false (nothing launched) when the matrix spans 4 GB
@@ -723,9 +734,10 @@ static bool vector_product(int opa, int opb, int64_t m, int64_t n, int64_t k, T 
     *st = workspace_get(stream, wsb, &lease, &ws);
     if (*st != EH_SUCCESS) return true;
   }
+  unsigned* tickets = gemv_tickets(g, stream, lease);
   KernelTimer t(EH_KC_GEMV, stream);
   hipError_t e = launch_gemv<T>(g, trans, rows, (int)k, alpha, mat, ldm, (uint32_t)(extent - 64 * sizeof(T)), x, incx,
-                                beta, C, incy, ws, stream);
+                                beta, C, incy, ws, tickets, stream);
   *st = e == hipSuccess ? EH_SUCCESS : hip_fail(e, "gemv launch");
   return true;
 }
@@ -856,9 +868,10 @@ static eh_status gemv_run(bool trans, int64_t rows, int64_t k, T alpha, const T*
     eh_status st = workspace_get(s, wsb, &lease, &ws);
     if (st != EH_SUCCESS) return st;
   }
+  unsigned* tickets = gemv_tickets(g, s, lease);
   KernelTimer t(EH_KC_GEMV, s);
   hipError_t e = launch_gemv<T>(g, trans, (int)rows, (int)k, alpha, A, lda, (uint32_t)(extent - 64 * sizeof(T)), x, incx,
-                                beta, y, incy, ws, s);
+                                beta, y, incy, ws, tickets, s);
   return e == hipSuccess ? EH_SUCCESS : hip_fail(e, "gemv launch");
 }
 

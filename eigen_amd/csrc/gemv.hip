@@ -11,14 +11,14 @@
 //   gemv_n_kernel  op(A)(i,k) = A[i + k*lda] (rows contiguous): each thread
 //                  owns 16 contiguous bytes of rows and walks k, the vector
 //                  element of each k being wave-uniform (scalar loads);
-//   gemv_t_kernel  op(A)(i,k) = A[k + i*lda] (k contiguous): each wave owns
-//                  eight rows, lanes read 16-byte chunks along k and the
-//                  vector chunk once for all eight rows, then reduce across
-//                  the wave.
+//   gemv_t_kernel  op(A)(i,k) = A[k + i*lda] (k contiguous): each wave walks
+//                  one row (or four short ones), lanes reading 16-byte chunks
+//                  along k against x in LDS, then reduces across the wave.
 //
 // Both split K over a second grid dimension when the rows alone cannot fill
-// the chip; partial sums go to the workspace and a reduction kernel applies
-// alpha/beta in a fixed order (deterministic).  Operands are read through
+// the chip; partial sums go to the workspace and are added in a fixed order
+// (deterministic), by a reduction kernel or, for Aᵀx where the caller has
+// tickets to give, by the last workgroup of each row block.  Operands are read through
 // raw buffer resources: reads past the end of the matrix return zero and
 // rows past m only feed outputs that are never stored.
 #include <hip/hip_runtime.h>
@@ -38,21 +38,58 @@ struct GemvParams {
   int m, k, k_per_split;
   uint32_t bytesA;  // extent of A from its base pointer (< 2^32, checked on the host)
   T alpha, beta;
+  unsigned* tickets;  // with W: one zero word per row block, or nullptr (gemv_reduce_kernel follows)
 };
 
+// Partial sums carry the device scope: another workgroup of this launch, on
+// any XCD, may add them up.
 template <typename T>
 __device__ inline void gemv_store(const GemvParams<T>& p, int i, T acc, int z) {
   if (p.W) {
-    p.W[(int64_t)z * p.m + i] = acc;
+    __hip_atomic_store(&p.W[(int64_t)z * p.m + i], acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
     T* dst = p.y + (int64_t)i * p.incy;
     *dst = (p.beta == T(0)) ? p.alpha * acc : fma_t(p.alpha, acc, p.beta * *dst);
   }
 }
 
-// Rows per wave of gemv_t_kernel: eight (against four) read the vector
-// chunk once per eight rows, 16384^2 FP64 A^T x 387 -> 352 us (FP32 equal).
-constexpr int kGemvRowsPerWave = 8;
+// y from the partial sums of row i, in split order; loads issued sixteen at a
+// time so that a long split list costs splits/16 memory latencies, not splits.
+template <typename T>
+__device__ inline void gemv_add_splits(const GemvParams<T>& p, int i, int splits) {
+  T s = T(0);
+  for (int z = 0; z < splits; z += 16) {
+    T v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      v[u] = __hip_atomic_load(&p.W[(int64_t)min(z + u, splits - 1) * p.m + i], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s = z + u < splits ? s + v[u] : s;
+  }
+  T* dst = p.y + (int64_t)i * p.incy;
+  *dst = (p.beta == T(0)) ? p.alpha * s : fma_t(p.alpha, s, p.beta * *dst);
+}
+
+// After a workgroup's partial sums: the last one of the row block to get here
+// adds the block's rows [i0, i1) up, in place of a second launch.  Aᵀx only: Ax
+// has few row blocks and many splits, and one workgroup adding them took longer
+// than a launch (FP64 300 x 12000: 20.7 against 18.1 us).
+template <typename T>
+__device__ inline void gemv_finish(const GemvParams<T>& p, int i0, int i1) {
+  if (!p.tickets) return;
+  __shared__ int last;
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's partial sums have reached memory
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = atomicAdd(&p.tickets[blockIdx.x], 1u) == gridDim.y - 1;
+    if (last) __hip_atomic_store(&p.tickets[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!last) return;
+  for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) gemv_add_splits(p, i, gridDim.y);
+}
+
 // k unroll of gemv_n_kernel (loads in flight per thread): 16 for FP64
 // (16384^2: 370 -> 362 us), 8 for FP32 (16 measured 2% slower).
 __host__ __device__ constexpr int gemv_n_unroll(int es) { return es == 8 ? 16 : 8; }
@@ -106,80 +143,141 @@ __device__ inline T wave_sum(T v) {
   return v;
 }
 
-// 4 waves x kGemvRowsPerWave rows per workgroup; each lane covers EPT
-// consecutive k of a 64*EPT chunk; k range of split blockIdx.y.
-template <typename T>
-__global__ void __launch_bounds__(256) gemv_t_kernel(GemvParams<T> p) {
+// Eight waves; the workgroup's rows [blockIdx.x * rows, + rows) over the k range
+// of split blockIdx.y, whose part of x lies in LDS.  A wave walks RB rows at a
+// time, each a contiguous stream of 1 KB loads, RB*U of them in flight: of one
+// row when the range is long, of four when it is short.  HBM bound.  Against
+// eight rows of 1 KB per wave with x read from L1, K split only by doubling:
+// FP64 6000 x 4001 43 -> 38 us (5.1 TB/s, matrix not in cache), 2000 x 2500 38
+// -> 12, 16384 x 256 25 -> 12, 8192 x 16384 216 -> 185 (5.8 TB/s), FP32 16000 x
+// 2500 35 -> 34; 16384^2, which fitted that form exactly, 351 -> 361.
+constexpr int kGemvTWaves = 8;
+constexpr int kGemvTBytes = 32768;  // of x in LDS: four workgroups per CU, whole batches of U chunks
+template <typename T, int RB, int U>
+__global__ void __launch_bounds__(64 * kGemvTWaves, 8) gemv_t_kernel(GemvParams<T> p, int rows) {
   constexpr int EPT = 16 / sizeof(T);
-  constexpr int RW = kGemvRowsPerWave;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int r0 = (blockIdx.x * 4 + wave) * RW;
+  constexpr int CH = 64 * EPT;  // elements of one load of a wave
+  __shared__ __attribute__((aligned(16))) T xs[kGemvTBytes / sizeof(T)];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int z = blockIdx.y;
-  const int kb = z * p.k_per_split, ke = min(p.k, kb + p.k_per_split);
+  const int kb = z * p.k_per_split, len = min(p.k - kb, p.k_per_split);
+  const int chunks = (len + CH - 1) / CH;
+  for (int i = threadIdx.x; i < (chunks + U - 1) / U * U * CH; i += 64 * kGemvTWaves)
+    xs[i] = i < len ? p.x[(int64_t)(kb + i) * p.incx] : T(0);
+  __syncthreads();
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, p.bytesA);
-  uint32_t vo[RW];
+  const int i0 = blockIdx.x * rows, i1 = min(p.m, i0 + rows);
+  auto load = [&](int r, int c, u32x4(&v)[RB][U]) {
 #pragma unroll
-  for (int r = 0; r < RW; ++r) vo[r] = (uint32_t)(((uint64_t)(r0 + r) * p.lda + lane * EPT) * sizeof(T));
-  T acc[RW];
+    for (int b = 0; b < RB; ++b) {
+      const uint32_t vo = (uint32_t)(((uint64_t)min(r + b, p.m - 1) * p.lda + lane * EPT) * sizeof(T));
 #pragma unroll
-  for (int r = 0; r < RW; ++r) acc[r] = T(0);
-  for (int k0 = kb; k0 < ke; k0 += 64 * EPT) {
-    const int kl = k0 + lane * EPT;
-    T xv[EPT];
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) xv[e] = kl + e < ke ? p.x[(int64_t)(kl + e) * p.incx] : T(0);
-#pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      const u32x4 v = buf_load16(rA, vo[r], (uint32_t)((uint64_t)k0 * sizeof(T)));
-      const T* a = reinterpret_cast<const T*>(&v);
-      // elements past ke (next row's data or the next split's) meet x = 0
-      // only if they are finite; select them away instead
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) acc[r] = fma_t(kl + e < ke ? a[e] : T(0), xv[e], acc[r]);
+      for (int u = 0; u < U; ++u)
+        v[b][u] = buf_load16(rA, vo, (uint32_t)((uint64_t)(kb + min(c + u, chunks - 1) * CH) * sizeof(T)));
     }
-  }
+  };
+  T acc[RB][EPT] = {};
+  // every wave starts its rows at another batch of the range: rows a power of
+  // two apart would otherwise all be read at one memory channel's addresses
+  const int batches = (chunks + U - 1) / U;
+  const int c0 = (int)((blockIdx.x * kGemvTWaves + wave) % batches) * U;
+  int r = i0 + wave * RB, c = c0;
+  while (r < i1) {
+    u32x4 v[RB][U];
+    load(r, c, v);
+    const int cn = c + U >= chunks ? 0 : c + U;
+    const bool row_ends = cn == c0;
+    const int rn = row_ends ? r + kGemvTWaves * RB : r;
+    if ((c + U) * CH > len) {
+      // elements past the range (the next row's data, the next split's, a
+      // repeated chunk) meet x = 0 only if they are finite; select them away
 #pragma unroll
-  for (int r = 0; r < RW; ++r) {
-    const T s = wave_sum(acc[r]);
-    if (lane == 0 && r0 + r < p.m) gemv_store(p, r0 + r, s, z);
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int e = 0; e < EPT; ++e) {
+            T* a = reinterpret_cast<T*>(&v[b][u]);
+            a[e] = (c + u) * CH + lane * EPT + e < len ? a[e] : T(0);
+          }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const u32x4 xv = *reinterpret_cast<const u32x4*>(&xs[(c + u) * CH + lane * EPT]);
+#pragma unroll
+      for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int e = 0; e < EPT; ++e)
+          acc[b][e] = fma_t(reinterpret_cast<const T*>(&v[b][u])[e], reinterpret_cast<const T*>(&xv)[e], acc[b][e]);
+    }
+    if (row_ends) {
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        T s = acc[b][0];
+#pragma unroll
+        for (int e = 1; e < EPT; ++e) s += acc[b][e];
+        s = wave_sum(s);
+        if (lane == 0 && r + b < i1) gemv_store(p, r + b, s, z);
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) acc[b][e] = T(0);
+      }
+    }
+    r = rn;
+    c = cn;
   }
+  gemv_finish(p, i0, i1);
 }
 
 template <typename T>
 __global__ void __launch_bounds__(256) gemv_reduce_kernel(GemvParams<T> p, int splits) {
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < p.m; i += gridDim.x * 256) {
-    // partials summed in split order; loads issued eight at a time so that a
-    // long split list costs splits/8 memory latencies, not splits
-    T s = T(0);
-    int z = 0;
-    for (; z + 8 <= splits; z += 8) {
-      T v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = p.W[(int64_t)(z + u) * p.m + i];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
-    }
-    for (; z < splits; ++z) s += p.W[(int64_t)z * p.m + i];
-    T* dst = p.y + (int64_t)i * p.incy;
-    *dst = (p.beta == T(0)) ? p.alpha * s : fma_t(p.alpha, s, p.beta * *dst);
-  }
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < p.m; i += gridDim.x * 256) gemv_add_splits(p, i, splits);
 }
 
-// Grid of a matrix-vector product: row blocks, and splits of K so that the
-// grid has at least ~2048 (Aᵀx) or ~256 (Ax) workgroups' worth of streaming,
-// each split a whole number of chunks of at least `min_k` columns.  Ax reads
-// fastest with one long-running workgroup per CU: each then streams long runs
-// of its columns, where 2048 shorter workgroups measured 10-20% slower.
+// Grid of a matrix-vector product: row blocks, and splits of K.
+//
+// Aᵀx: splits whose part of x fits in LDS, in whole batches of loads; among
+// them, and one or two rows (or groups of rows) per wave, the plan whose rounds
+// of resident workgroups (four per CU) stream the fewest bytes, x's part
+// counted as one row and a workgroup's start as 16 KB.  More rows per workgroup
+// leave the last round uneven (16384^2 FP64: 361, 363, 368 us with 16, 32, 64).
+static GemvPlan gemv_t_plan(int m, int k, int es) {
+  constexpr int kGroups = 1024;
+  const int chunk = 64 * 16 / es;
+  GemvPlan best{};
+  double best_cost = 0;
+  const int smin = (int)(((int64_t)k * es + kGemvTBytes - 1) / kGemvTBytes);
+  for (int s = smin; s == smin || (s < smin + 16 && (int64_t)k * es >= (int64_t)s * 4096); ++s) {
+    int64_t per = ((int64_t)k + s - 1) / s;
+    GemvPlan g{};
+    g.batch = per >= 6 * chunk ? 1 : 4;
+    const int whole = 8 * chunk / g.batch;  // whole batches: 8 KB of a row, or 2 KB
+    per = (per + whole - 1) / whole * whole;
+    g.per = (int)per;
+    g.splits = (int)(((int64_t)k + per - 1) / per);
+    const int step = kGemvTWaves * g.batch;
+    for (g.rows = step; g.rows <= 2 * step; g.rows += step) {
+      g.blocks = (m + g.rows - 1) / g.rows;
+      const int64_t rounds = ((int64_t)g.blocks * g.splits + kGroups - 1) / kGroups;
+      const double cost = (double)rounds * ((g.rows + 1.0) * (double)per * es + 16384.0);
+      if (best.blocks == 0 || cost < best_cost) {
+        best = g;
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
+// Ax: about 256 workgroups' worth of streaming, one long-running workgroup per
+// CU: each then streams long runs of its columns, where 2048 shorter workgroups
+// measured 10-20% slower.
 GemvPlan gemv_plan(bool trans, int m, int k, int es) {
-  const int ept = 16 / es;
+  if (trans) return gemv_t_plan(m, k, es);
+  const int ept = 16 / es, chunk = gemv_n_unroll(es);
   GemvPlan g{};
-  g.blocks = trans ? (m + 4 * kGemvRowsPerWave - 1) / (4 * kGemvRowsPerWave) : (m + 256 * ept - 1) / (256 * ept);
-  const int chunk = trans ? 64 * ept : gemv_n_unroll(es);
-  const int min_k = trans ? 4 * chunk : 64;
-  const int64_t target = trans ? 2048 : 256;
+  g.blocks = (m + 256 * ept - 1) / (256 * ept);
   int s = 1;
-  while ((int64_t)g.blocks * s < target && k / (2 * s) >= min_k && s < 256) s *= 2;
+  while ((int64_t)g.blocks * s < 256 && k / (2 * s) >= 64 && s < 256) s *= 2;
   int64_t per = ((int64_t)k + s - 1) / s;
   per = (per + chunk - 1) / chunk * chunk;
   g.per = (int)per;
@@ -195,7 +293,7 @@ size_t gemv_workspace_bytes(const GemvPlan& g, int m, int es) {
 template <typename T>
 hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, const T* A, int64_t lda,
                        uint32_t bytesA, const T* x, int64_t incx, T beta, T* y, int64_t incy, void* workspace,
-                       hipStream_t s) {
+                       unsigned* tickets, hipStream_t s) {
   GemvParams<T> p{};
   p.A = A;
   p.x = x;
@@ -210,13 +308,16 @@ hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, con
   p.beta = beta;
   p.k_per_split = g.per;
   p.W = g.splits > 1 ? static_cast<T*>(workspace) : nullptr;
+  p.tickets = trans && g.splits > 1 ? tickets : nullptr;
   dim3 grid((unsigned)g.blocks, (unsigned)g.splits);
-  if (trans)
-    hipLaunchKernelGGL(gemv_t_kernel<T>, grid, dim3(256), 0, s, p);
+  if (trans && g.batch == 1)
+    hipLaunchKernelGGL((gemv_t_kernel<T, 1, 8>), grid, dim3(64 * kGemvTWaves), 0, s, p, g.rows);
+  else if (trans)
+    hipLaunchKernelGGL((gemv_t_kernel<T, 4, 2>), grid, dim3(64 * kGemvTWaves), 0, s, p, g.rows);
   else
     hipLaunchKernelGGL(gemv_n_kernel<T>, grid, dim3(256), 0, s, p);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || g.splits == 1) return e;
+  if (e != hipSuccess || g.splits == 1 || p.tickets) return e;
   int64_t rb = (m + 255) / 256;
   if (rb > 65536) rb = 65536;
   hipLaunchKernelGGL(gemv_reduce_kernel<T>, dim3((unsigned)rb), dim3(256), 0, s, p, g.splits);
@@ -224,8 +325,9 @@ hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, con
 }
 
 template hipError_t launch_gemv<float>(const GemvPlan&, bool, int, int, float, const float*, int64_t, uint32_t,
-                                       const float*, int64_t, float, float*, int64_t, void*, hipStream_t);
+                                       const float*, int64_t, float, float*, int64_t, void*, unsigned*, hipStream_t);
 template hipError_t launch_gemv<double>(const GemvPlan&, bool, int, int, double, const double*, int64_t, uint32_t,
-                                        const double*, int64_t, double, double*, int64_t, void*, hipStream_t);
+                                        const double*, int64_t, double, double*, int64_t, void*, unsigned*,
+                                        hipStream_t);
 
 }  // namespace eh

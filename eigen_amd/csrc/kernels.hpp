@@ -68,13 +68,16 @@ hipError_t launch_strided_combine(const T* W, int M, int N, T* C, int64_t incc, 
 // needs gemv_workspace_bytes of workspace for the partial sums.
 struct GemvPlan {
   int blocks, splits, per;
+  int rows, batch;  // A^T x: rows of a workgroup, rows a wave walks together
 };
+// tickets (one zero word per row block, or nullptr): the last workgroup of a
+// row block adds its partial sums and no second launch follows.
 GemvPlan gemv_plan(bool trans, int m, int k, int es);
 size_t gemv_workspace_bytes(const GemvPlan& g, int m, int es);
 template <typename T>
 hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, const T* A, int64_t lda,
                        uint32_t bytesA, const T* x, int64_t incx, T beta, T* y, int64_t incy, void* workspace,
-                       hipStream_t s);
+                       unsigned* tickets, hipStream_t s);
 
 // Dense form of the n x n matrix stored in one triangle of A (lower: i >= j):
 // sym mirrors the stored triangle, otherwise the other triangle is zero and

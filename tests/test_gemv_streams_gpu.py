@@ -1,0 +1,55 @@
+"""y = alpha*A^T*x + beta*y where its plan changes: x parts past the LDS tile,
+rows walked one at a time and four at a time, row blocks that end early, split
+K finished by the last workgroup (called twice, so tickets left uncleared would
+show) and, through a captured graph, by the reduction kernel; exact integers,
+NaN in the padding and between the vectors' elements."""
+import numpy as np
+import pytest
+import torch
+
+import eigen_amd as E
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,code", [(np.float32, E.F32), (np.float64, E.F64)])
+@pytest.mark.parametrize("m,n,pad,incx,incy", [
+    (1, 1, 0, 1, 1), (127, 3, 1, 2, 1), (129, 70, 0, 1, 3), (767, 33, 1, 1, 1), (1025, 257, 1, -1, 2), (4097, 300, 0, 1, 1),
+    (8193, 17, 1, 3, -1), (16385, 64, 1, 1, 1), (40001, 9, 3, 1, 1), (300, 16390, 0, 1, 1)])
+def test_gemv_t_exact(gpu, dtype, code, m, n, pad, incx, incy):
+    A = O.fill((m + pad, n), dtype, 1, O.INT, -3, 3)
+    A[m:] = np.nan
+    x, y = O.fill((m, 1), dtype, 2, O.INT, -3, 3)[:, 0], O.fill((n, 1), dtype, 3, O.INT, -3, 3)[:, 0]
+    want = 2.0 * (A[:m].astype(np.float64).T @ x) - y
+
+    def spread(v, inc):
+        s = np.full((len(v) - 1) * abs(inc) + 1, np.nan, dtype)
+        s[::abs(inc)] = v if inc > 0 else v[::-1]
+        return torch.from_numpy(s).cuda()
+
+    a, dx, y0 = torch.from_numpy(A.reshape(-1, order="F").copy()).cuda(), spread(x, incx), spread(y, incy)
+    dy = y0.clone()
+    call = lambda s=None: E.gemv(code, 1, m, n, 2.0, a, m + pad, dx, incx, -1.0, dy, incy, stream=s)  # noqa: E731
+
+    def check():
+        torch.cuda.synchronize()
+        got = dy.cpu().numpy()[::abs(incy)]
+        assert np.array_equal((got if incy > 0 else got[::-1]).astype(np.float64), want)
+
+    for _ in range(2):
+        dy.copy_(y0)
+        call()
+        check()
+    g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        call(s.cuda_stream)  # the stream's workspace exists before the capture
+        torch.cuda.synchronize()
+        g.capture_begin()
+        call(s.cuda_stream)
+        g.capture_end()
+    for _ in range(2):
+        dy.copy_(y0)
+        torch.cuda.synchronize()
+        g.replay()
+        check()
