@@ -656,18 +656,17 @@ static void launch_dense_t(eh_dtype dtype, const void* A, int64_t sa, const void
 // Products of at most 16 x 16 with depth at most 4 * KS (KS = 4, 8 or 16),
 // one wave each: a single 16 x 16 MFMA block (v_mfma_f32_16x16x4_f32 /
 // v_mfma_f64_16x16x4_f64) holds C^T = op(B)^T op(A)^T, so consecutive lanes
-// store consecutive rows of C.  Lane l feeds row / column l % 16 at depth
-// k0 + l / 16 of each 4-deep step; all KS steps are loaded up front from
-// clamped addresses inside the product and zeroed by selects past m, n or k,
-// so no load waits on another and none leaves the product.  A 32 x 32 tile
-// of the grouped kernel would spend 3/4 of its MFMAs and half its loads on
-// zeros for a 16 x 16 product: 20,000 FP64 16^3 products take 23.6 us here
-// against 30.8 us there (kernel events; 29.0 against 40.6 us per call, which
-// also saves the work-list kernel), FP32 18.7 against 24.9 us, 50,000 FP64
-// 8^3 30.2 against 47.1 us.  Deeper products stay on the grouped kernel,
-// whose 16-byte loads of k-contiguous slabs win there (FP32 beyond depth
-// 32, FP64 beyond 64): a loop over passes of 64 here measured 48% slower on
-// FP32 16x16x256 (225 against 152 us), 4% faster on FP64.
+// store consecutive rows of C.  Lane l feeds row / column l % 16; its k values
+// are consecutive in 16-byte runs (load_small), so that a k-contiguous operand
+// takes one load per run.  All KS steps are loaded up front from clamped
+// addresses inside the product, and zeroed past m, n or k only where they are
+// multiplied, so no load waits on another and none leaves the product.  HBM
+// bound: 20,000 FP64 16^3 products 23.6 us per call (5.2 TB/s; 28.3 with a
+// select after each load and one element per load), with A transposed 23.7
+// (33.8), FP32 13.6 (18.5), 50,000 FP64 8^3 21.7 (31.4); FP32 16x16x64 32.7
+// against 54.2 through the grouped kernel's 32x32 tiles, 16x16x36 22.8 against
+// 42.4.  Odd k reads a k-contiguous operand an element at a time (FP32
+// 16x16x63, A transposed: 55.5 against 59.6 there).
 template <typename T>
 struct Small16;
 template <>
@@ -687,32 +686,48 @@ struct Small16<double> {
   __device__ static int col(int r, int q) { return q + 4 * r; }
 };
 
-template <typename T, bool TA, bool TB, int KS>
+// Operand values of one lane: step EPC*c + e holds k = 4*EPC*c + EPC*q + e of
+// row r, so that a k-contiguous operand (VEC: k a multiple of EPC) is read 16
+// bytes at a time.
+template <typename T, bool KC, bool VEC, int KS>
+__device__ inline void load_small(const T* X, int64_t ld, int r, int k, int q, T (&v)[KS]) {
+  constexpr int EPC = 16 / sizeof(T);
+#pragma unroll
+  for (int c = 0; c < KS / EPC; ++c) {
+    const int kk = 4 * EPC * c + EPC * q;
+    if constexpr (KC && VEC) {
+      __builtin_memcpy(&v[EPC * c], X + min(kk, k - EPC) + (int64_t)r * ld, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) {
+        const int kc = min(kk + e, k - 1);
+        v[EPC * c + e] = KC ? X[kc + (int64_t)r * ld] : X[r + (int64_t)kc * ld];
+      }
+    }
+  }
+}
+
+template <typename T, bool TA, bool TB, int KS, bool VEC>
 __global__ void __launch_bounds__(256) small_batched_kernel(const T* __restrict__ A, int64_t lda, int64_t sa,
                                                             const T* __restrict__ B, int64_t ldb, int64_t sb,
                                                             T* __restrict__ C, int64_t ldc, int64_t sc, int m, int n,
                                                             int k, T alpha, T beta, int64_t count) {
   using S = Small16<T>;
+  constexpr int EPC = 16 / sizeof(T);
   const int64_t p = blockIdx.x * 4ll + (threadIdx.x >> 6);
   if (p >= count) return;
   const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
-  const T* Ap = A + p * sa;
-  const T* Bp = B + p * sb;
-  const int ic = min(r16, m - 1), jc = min(r16, n - 1);
   T a[KS], b[KS];
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    const int kk = 4 * s + q, kc = min(kk, k - 1);
-    const T va = TA ? Ap[kc + (int64_t)ic * lda] : Ap[ic + (int64_t)kc * lda];
-    const T vb = TB ? Bp[jc + (int64_t)kc * ldb] : Bp[kc + (int64_t)jc * ldb];
-    a[s] = (r16 < m && kk < k) ? va : T(0);
-    b[s] = (r16 < n && kk < k) ? vb : T(0);
-  }
+  load_small<T, TA, VEC, KS>(A + p * sa, lda, min(r16, m - 1), k, q, a);
+  load_small<T, !TB, VEC, KS>(B + p * sb, ldb, min(r16, n - 1), k, q, b);
   typename S::acc_t acc;
 #pragma unroll
   for (int r = 0; r < 4; ++r) acc[r] = T(0);
 #pragma unroll
-  for (int s = 0; s < KS; ++s) acc = S::mma(b[s], a[s], acc);
+  for (int s = 0; s < KS; ++s) {
+    const bool in = 4 * EPC * (s / EPC) + EPC * q + s % EPC < k;
+    acc = S::mma(in && r16 < n ? b[s] : T(0), in && r16 < m ? a[s] : T(0), acc);
+  }
   const bool row_in = r16 < m;
   T* Cp = C + p * sc + r16;
   if (beta != T(0)) {  // every C value of the lane read before the first store
@@ -735,8 +750,8 @@ __global__ void __launch_bounds__(256) small_batched_kernel(const T* __restrict_
   }
 }
 
-template <typename T, int KS>
-static void launch_small_t(bool ta, bool tb, const void* A, int64_t lda, int64_t sa, const void* B, int64_t ldb,
+template <typename T, int KS, bool VEC>
+static void launch_small_vec(bool ta, bool tb, const void* A, int64_t lda, int64_t sa, const void* B, int64_t ldb,
                            int64_t sb, void* C, int64_t ldc, int64_t sc, int m, int n, int k, T alpha, T beta,
                            int64_t count, hipStream_t s) {
   const dim3 grid((unsigned)((count + 3) / 4)), block(256);
@@ -744,17 +759,27 @@ static void launch_small_t(bool ta, bool tb, const void* A, int64_t lda, int64_t
   const T* b = static_cast<const T*>(B);
   T* c = static_cast<T*>(C);
   if (!ta && !tb)
-    hipLaunchKernelGGL((small_batched_kernel<T, false, false, KS>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, false, false, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
   else if (ta && !tb)
-    hipLaunchKernelGGL((small_batched_kernel<T, true, false, KS>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, true, false, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
   else if (!ta && tb)
-    hipLaunchKernelGGL((small_batched_kernel<T, false, true, KS>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, false, true, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
   else
-    hipLaunchKernelGGL((small_batched_kernel<T, true, true, KS>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, true, true, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
+}
+
+template <typename T, int KS>
+static void launch_small_t(bool ta, bool tb, const void* A, int64_t lda, int64_t sa, const void* B, int64_t ldb,
+                           int64_t sb, void* C, int64_t ldc, int64_t sc, int m, int n, int k, T alpha, T beta,
+                           int64_t count, hipStream_t s) {
+  if (k % (16 / (int)sizeof(T)) == 0)
+    launch_small_vec<T, KS, true>(ta, tb, A, lda, sa, B, ldb, sb, C, ldc, sc, m, n, k, alpha, beta, count, s);
+  else
+    launch_small_vec<T, KS, false>(ta, tb, A, lda, sa, B, ldb, sb, C, ldc, sc, m, n, k, alpha, beta, count, s);
 }
 
 }  // namespace eh
@@ -825,33 +850,28 @@ extern "C" eh_status eh_gemm_batched_strided(eh_dtype dtype, eh_op opa, eh_op op
   const double be = dtype == EH_F64 ? *static_cast<const double*>(beta) : *static_cast<const float*>(beta);
   const bool ta = opa != EH_OP_N, tb = opb != EH_OP_N;
   const bool reads = k > 0 && al != 0.0;
-  // one wave per product up to 16 x 16: FP64 to depth 64, FP32 to depth 32,
-  // in one pass of 4, 8 or 16 four-deep steps (a pass with steps past the
-  // depth still loads them: FP64 16x16x32 took 65.7 us with 16 steps, 37.5
-  // with 8; FP32 16x16x32 29.5 us against 33.4 through the grouped kernel,
-  // 16x16x64 with 16 steps 50 against 46 us there)
-  if (reads && m <= 16 && n <= 16 && k <= (dtype == EH_F64 ? 64 : 32)) {
+  // one wave per product up to 16 x 16 and depth 64, in one pass of 4, 8 or 16
+  // four-deep steps (a pass with steps past the depth still loads them: FP64
+  // 16x16x32 took 65.7 us with 16 steps, 37.5 with 8)
+  if (reads && m <= 16 && n <= 16 && k <= 64) {
     KernelTimer t(EH_KC_GROUPED, s);
-    if (dtype == EH_F64) {
-      const double a = *static_cast<const double*>(alpha), b = *static_cast<const double*>(beta);
+    auto launch = [&](auto zero) {
+      using T = decltype(zero);
+      const T a = *static_cast<const T*>(alpha), b = *static_cast<const T*>(beta);
       if (k <= 16)
-        launch_small_t<double, 4>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k,
-                                  a, b, count, s);
+        launch_small_t<T, 4>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k, a, b,
+                             count, s);
       else if (k <= 32)
-        launch_small_t<double, 8>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k,
-                                  a, b, count, s);
+        launch_small_t<T, 8>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k, a, b,
+                             count, s);
       else
-        launch_small_t<double, 16>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n,
-                                   (int)k, a, b, count, s);
-    } else {
-      const float a = *static_cast<const float*>(alpha), b = *static_cast<const float*>(beta);
-      if (k <= 16)
-        launch_small_t<float, 4>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k,
-                                 a, b, count, s);
-      else  // k <= 32
-        launch_small_t<float, 8>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k,
-                                 a, b, count, s);
-    }
+        launch_small_t<T, 16>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k, a,
+                              b, count, s);
+    };
+    if (dtype == EH_F64)
+      launch(0.0);
+    else
+      launch(0.0f);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? EH_SUCCESS : hip_fail(e, "small batched launch");
   }
