@@ -653,9 +653,9 @@ static void launch_dense_t(eh_dtype dtype, const void* A, int64_t sa, const void
                        *static_cast<const float*>(alpha), *static_cast<const float*>(beta), count);
 }
 
-// Products of at most 16 x 16 with depth at most 4 * KS (KS = 4, 8 or 16),
-// one wave each: a single 16 x 16 MFMA block (v_mfma_f32_16x16x4_f32 /
-// v_mfma_f64_16x16x4_f64) holds C^T = op(B)^T op(A)^T, so consecutive lanes
+// Products of at most 16R x 16R (R = 1, 2) with depth at most 4 * KS, one wave
+// each: R x R blocks of 16 x 16 (v_mfma_f32_16x16x4_f32 /
+// v_mfma_f64_16x16x4_f64) hold C^T = op(B)^T op(A)^T, so consecutive lanes
 // store consecutive rows of C.  Lane l feeds row / column l % 16; its k values
 // are consecutive in 16-byte runs (load_small), so that a k-contiguous operand
 // takes one load per run.  All KS steps are loaded up front from clamped
@@ -665,8 +665,7 @@ static void launch_dense_t(eh_dtype dtype, const void* A, int64_t sa, const void
 // select after each load and one element per load), with A transposed 23.7
 // (33.8), FP32 13.6 (18.5), 50,000 FP64 8^3 21.7 (31.4); FP32 16x16x64 32.7
 // against 54.2 through the grouped kernel's 32x32 tiles, 16x16x36 22.8 against
-// 42.4.  Odd k reads a k-contiguous operand an element at a time (FP32
-// 16x16x63, A transposed: 55.5 against 59.6 there).
+// 42.4.
 template <typename T>
 struct Small16;
 template <>
@@ -687,15 +686,17 @@ struct Small16<double> {
 };
 
 // Operand values of one lane: step EPC*c + e holds k = 4*EPC*c + EPC*q + e of
-// row r, so that a k-contiguous operand (VEC: k a multiple of EPC) is read 16
-// bytes at a time.
-template <typename T, bool KC, bool VEC, int KS>
+// row r, so that a k-contiguous operand is read 16 bytes at a time.  A run that
+// ends past k is read where it ends at k and moved into place (shift_small)
+// when it is multiplied.  VEC: 0 = k shorter than a run (element by element), 1
+// = k a multiple of a run, 2 = any other k.
+template <typename T, bool KC, int VEC, int KS>
 __device__ inline void load_small(const T* X, int64_t ld, int r, int k, int q, T (&v)[KS]) {
   constexpr int EPC = 16 / sizeof(T);
 #pragma unroll
   for (int c = 0; c < KS / EPC; ++c) {
     const int kk = 4 * EPC * c + EPC * q;
-    if constexpr (KC && VEC) {
+    if constexpr (KC && VEC > 0) {
       __builtin_memcpy(&v[EPC * c], X + min(kk, k - EPC) + (int64_t)r * ld, 16);
     } else {
 #pragma unroll
@@ -706,8 +707,22 @@ __device__ inline void load_small(const T* X, int64_t ld, int r, int k, int q, T
     }
   }
 }
+template <typename T, bool KC, int VEC, int KS>
+__device__ inline void shift_small(int k, int q, T (&v)[KS]) {
+  constexpr int EPC = 16 / sizeof(T);
+  if constexpr (KC && VEC == 2) {
+#pragma unroll
+    for (int c = 0; c < KS / EPC; ++c) {
+      const int d = 4 * EPC * c + EPC * q - (k - EPC);  // the run was read d elements early
+#pragma unroll
+      for (int e = 0; e < EPC; ++e)
+#pragma unroll
+        for (int x = 1; e + x < EPC; ++x) v[EPC * c + e] = d == x ? v[EPC * c + e + x] : v[EPC * c + e];
+    }
+  }
+}
 
-template <typename T, bool TA, bool TB, int KS, bool VEC>
+template <typename T, bool TA, bool TB, int KS, int VEC, int R>
 __global__ void __launch_bounds__(256) small_batched_kernel(const T* __restrict__ A, int64_t lda, int64_t sa,
                                                             const T* __restrict__ B, int64_t ldb, int64_t sb,
                                                             T* __restrict__ C, int64_t ldc, int64_t sc, int m, int n,
@@ -717,40 +732,56 @@ __global__ void __launch_bounds__(256) small_batched_kernel(const T* __restrict_
   const int64_t p = blockIdx.x * 4ll + (threadIdx.x >> 6);
   if (p >= count) return;
   const int lane = threadIdx.x & 63, r16 = lane & 15, q = lane >> 4;
-  T a[KS], b[KS];
-  load_small<T, TA, VEC, KS>(A + p * sa, lda, min(r16, m - 1), k, q, a);
-  load_small<T, !TB, VEC, KS>(B + p * sb, ldb, min(r16, n - 1), k, q, b);
-  typename S::acc_t acc;
+  T a[R][KS], b[R][KS];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) acc[r] = T(0);
+  for (int x = 0; x < R; ++x) {
+    load_small<T, TA, VEC, KS>(A + p * sa, lda, min(16 * x + r16, m - 1), k, q, a[x]);
+    load_small<T, !TB, VEC, KS>(B + p * sb, ldb, min(16 * x + r16, n - 1), k, q, b[x]);
+  }
+#pragma unroll
+  for (int x = 0; x < R; ++x) {
+    shift_small<T, TA, VEC, KS>(k, q, a[x]);
+    shift_small<T, !TB, VEC, KS>(k, q, b[x]);
+  }
+  typename S::acc_t acc[R][R] = {};  // acc[y][x]: rows 16x.., columns 16y.. of C
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
     const bool in = 4 * EPC * (s / EPC) + EPC * q + s % EPC < k;
-    acc = S::mma(in && r16 < n ? b[s] : T(0), in && r16 < m ? a[s] : T(0), acc);
-  }
-  const bool row_in = r16 < m;
-  T* Cp = C + p * sc + r16;
-  if (beta != T(0)) {  // every C value of the lane read before the first store
-    T c[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int j = S::col(r, q);
-      c[r] = row_in && j < n ? Cp[(int64_t)j * ldc] : T(0);
+    for (int y = 0; y < R; ++y)
+#pragma unroll
+      for (int x = 0; x < R; ++x)
+        acc[y][x] = S::mma(in && 16 * y + r16 < n ? b[y][s] : T(0), in && 16 * x + r16 < m ? a[x][s] : T(0), acc[y][x]);
+  }
+#pragma unroll
+  for (int x = 0; x < R; ++x) {
+    const bool row_in = 16 * x + r16 < m;
+    T* Cp = C + p * sc + 16 * x + r16;
+#pragma unroll
+    for (int y = 0; y < R; ++y) {
+      if (beta != T(0)) {  // every C value of the block read before its first store
+        T c[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = 16 * y + S::col(r, q);
+          c[r] = row_in && j < n ? Cp[(int64_t)j * ldc] : T(0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[y][x][r] = fma_t(alpha, acc[y][x][r], beta * c[r]);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[y][x][r] *= alpha;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = 16 * y + S::col(r, q);
+        if (row_in && j < n) Cp[(int64_t)j * ldc] = acc[y][x][r];
+      }
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[r] = fma_t(alpha, acc[r], beta * c[r]);
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[r] *= alpha;
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int j = S::col(r, q);
-    if (row_in && j < n) Cp[(int64_t)j * ldc] = acc[r];
   }
 }
 
-template <typename T, int KS, bool VEC>
+template <typename T, int KS, int VEC, int R>
 static void launch_small_vec(bool ta, bool tb, const void* A, int64_t lda, int64_t sa, const void* B, int64_t ldb,
                            int64_t sb, void* C, int64_t ldc, int64_t sc, int m, int n, int k, T alpha, T beta,
                            int64_t count, hipStream_t s) {
@@ -759,16 +790,16 @@ static void launch_small_vec(bool ta, bool tb, const void* A, int64_t lda, int64
   const T* b = static_cast<const T*>(B);
   T* c = static_cast<T*>(C);
   if (!ta && !tb)
-    hipLaunchKernelGGL((small_batched_kernel<T, false, false, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, false, false, KS, VEC, R>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
   else if (ta && !tb)
-    hipLaunchKernelGGL((small_batched_kernel<T, true, false, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, true, false, KS, VEC, R>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
   else if (!ta && tb)
-    hipLaunchKernelGGL((small_batched_kernel<T, false, true, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, false, true, KS, VEC, R>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
   else
-    hipLaunchKernelGGL((small_batched_kernel<T, true, true, KS, VEC>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
+    hipLaunchKernelGGL((small_batched_kernel<T, true, true, KS, VEC, R>), grid, block, 0, s, a, lda, sa, b, ldb, sb, c, ldc,
                        sc, m, n, k, alpha, beta, count);
 }
 
@@ -776,10 +807,12 @@ template <typename T, int KS>
 static void launch_small_t(bool ta, bool tb, const void* A, int64_t lda, int64_t sa, const void* B, int64_t ldb,
                            int64_t sb, void* C, int64_t ldc, int64_t sc, int m, int n, int k, T alpha, T beta,
                            int64_t count, hipStream_t s) {
-  if (k % (16 / (int)sizeof(T)) == 0)
-    launch_small_vec<T, KS, true>(ta, tb, A, lda, sa, B, ldb, sb, C, ldc, sc, m, n, k, alpha, beta, count, s);
-  else
-    launch_small_vec<T, KS, false>(ta, tb, A, lda, sa, B, ldb, sb, C, ldc, sc, m, n, k, alpha, beta, count, s);
+  constexpr int EPC = 16 / sizeof(T);
+  const bool one = m <= 16 && n <= 16;
+  auto f = k < EPC        ? (one ? launch_small_vec<T, KS, 0, 1> : launch_small_vec<T, KS, 0, 2>)
+           : k % EPC == 0 ? (one ? launch_small_vec<T, KS, 1, 1> : launch_small_vec<T, KS, 1, 2>)
+                          : (one ? launch_small_vec<T, KS, 2, 1> : launch_small_vec<T, KS, 2, 2>);
+  f(ta, tb, A, lda, sa, B, ldb, sb, C, ldc, sc, m, n, k, alpha, beta, count, s);
 }
 
 }  // namespace eh
@@ -850,23 +883,27 @@ extern "C" eh_status eh_gemm_batched_strided(eh_dtype dtype, eh_op opa, eh_op op
   const double be = dtype == EH_F64 ? *static_cast<const double*>(beta) : *static_cast<const float*>(beta);
   const bool ta = opa != EH_OP_N, tb = opb != EH_OP_N;
   const bool reads = k > 0 && al != 0.0;
-  // one wave per product up to 16 x 16 and depth 64, in one pass of 4, 8 or 16
-  // four-deep steps (a pass with steps past the depth still loads them: FP64
-  // 16x16x32 took 65.7 us with 16 steps, 37.5 with 8)
-  if (reads && m <= 16 && n <= 16 && k <= 64) {
+  // one wave per product up to 32 x 32 and depth 64, in one pass of as few
+  // four-deep steps as hold the depth, in whole 16-byte runs (steps past the
+  // depth are still loaded: FP64 16x16x32 took 65.7 us with 16 steps, 37.5 with
+  // 8).  Between 16 and 32, against the grouped kernel, which stages nothing
+  // either but runs a work list: FP64 5000 32^3 27.0 / 35.3 us, FP32 15.6 /
+  // 23.8, FP64 20000 30x6x10 21.4 / 38.2, 8000 24x31x17 30.5 / 36.1.
+  if (reads && m <= 32 && n <= 32 && k <= 64) {
     KernelTimer t(EH_KC_GROUPED, s);
     auto launch = [&](auto zero) {
       using T = decltype(zero);
       const T a = *static_cast<const T*>(alpha), b = *static_cast<const T*>(beta);
+      auto f = launch_small_t<T, 16>;
       if (k <= 16)
-        launch_small_t<T, 4>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k, a, b,
-                             count, s);
+        f = launch_small_t<T, 4>;
+      else if (sizeof(T) == 8 && k <= 24)
+        f = launch_small_t<T, sizeof(T) == 8 ? 6 : 8>;
       else if (k <= 32)
-        launch_small_t<T, 8>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k, a, b,
-                             count, s);
-      else
-        launch_small_t<T, 16>(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k, a,
-                              b, count, s);
+        f = launch_small_t<T, 8>;
+      else if (k <= 48)
+        f = launch_small_t<T, 12>;
+      f(ta, tb, A, lda, stride_a, B, ldb, stride_b, C, ldc, stride_c, (int)m, (int)n, (int)k, a, b, count, s);
     };
     if (dtype == EH_F64)
       launch(0.0);
