@@ -209,8 +209,8 @@ eh_status trsm_right(const Tri<T>& E, int64_t d, int64_t sz, T* B, int64_t ldb, 
 // ---- TRMM --------------------------------------------------------------------
 // Real types: ranges up to kTrmmLeafReal multiply a copy of their part of B
 // by the triangle itself in one launch (tri_product).  FP32 1500 x 1100 from
-// the right: 51 us, against 180 through 256-row dense leaves (17 launches);
-// FP64 8192 x 8192: 9.4 against 9.9 ms.
+// the right: 48 us, against 180 through 256-row dense leaves (17 launches);
+// FP64 8192 x 8192: 9.3 against 9.9 ms.
 // Complex types, and triangles past 32-bit addressing, expand dense leaves.
 constexpr int64_t kTrmmLeaf = 256;
 constexpr int64_t kTrmmLeafReal = 2048;

