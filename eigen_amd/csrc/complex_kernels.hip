@@ -9,8 +9,9 @@
 //   C3 (2m x n real):   rows 2i, 2i+1 of column j are Re, Im of C(i, j),
 // C3 = A3*B3 + beta*C3 is the complex product with alpha folded in and a real
 // beta.  C3 is C itself viewed as a real matrix (leading dimension 2*ldc), and
-// so is B3 when op(B) = B (leading dimension 2*ldb): only A, and B when
-// transposed or conjugated, are repacked.  This is the 4M scheme (four real
+// so is B3 when op(B) = B (leading dimension 2*ldb): only B when transposed
+// or conjugated is repacked, and A where the product kernel does not form A3's
+// blocks itself (complex_gemm.cpp).  This is the 4M scheme (four real
 // products per complex one, the same 8mnk flops) fused into a single large
 // product; Eigen's complex GEBP instead keeps separate real and imaginary
 // accumulators per micro-panel (GeneralBlockPanelKernel.h:631-1050).

@@ -11,7 +11,8 @@
 // before anything is launched.  The array is shared by every call on the
 // GPU: calls that overlap in time on one GPU race on it (the caller
 // serialises them, e.g. by using one stream).  Nothing in it needs to start
-// at zero: every kernel writes each scratch element it later reads.
+// at zero: every kernel writes each scratch element it later reads, and the
+// tickets of a balanced product are cleared by a launch before it.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
