@@ -90,12 +90,26 @@ __device__ inline void gemv_finish(const GemvParams<T>& p, int i0, int i1) {
   for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) gemv_add_splits(p, i, gridDim.y);
 }
 
+// A's loads, with the non-temporal hint (NT) when the matrix will not be found
+// in the 256 MB last-level cache by the next call anyway: it then reads 10%
+// faster (16384^2 FP64 A^T x 369 -> 331 us, Ax 361 -> 328; FP32 A^T x 204 ->
+// 181).  Below 256 MB a matrix may stay there between calls and be read faster
+// without the hint: A^T x of 192 MB 37.6 -> 34.2 us when it does not, 31.0 ->
+// 33.9 when it does, Ax 39.5 -> 37.6 and 31.7 -> 35.7.  So A^T x takes the hint
+// from half that cache on, which survives only if little else is used, Ax from
+// all of it; small matrices lose either way (Ax 500 x 4000 11.8 -> 17.3).
+template <bool NT>
+__device__ inline u32x4 matrix_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+  return NT ? buf_load16_stream(r, voff, soff) : buf_load16(r, voff, soff);
+}
+static bool gemv_streams(bool trans, uint32_t bytes) { return bytes >= (trans ? 128u : 256u) << 20; }
+
 // k unroll of gemv_n_kernel (loads in flight per thread): 16 for FP64
 // (16384^2: 370 -> 362 us), 8 for FP32 (16 measured 2% slower).
 __host__ __device__ constexpr int gemv_n_unroll(int es) { return es == 8 ? 16 : 8; }
 
 // 256 threads x EPT rows; k range of split blockIdx.y, unrolled by U.
-template <typename T>
+template <typename T, bool NT>
 __global__ void __launch_bounds__(256) gemv_n_kernel(GemvParams<T> p) {
   constexpr int EPT = 16 / sizeof(T);
   constexpr int U = gemv_n_unroll((int)sizeof(T));
@@ -113,7 +127,7 @@ __global__ void __launch_bounds__(256) gemv_n_kernel(GemvParams<T> p) {
     T xv[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      v[u] = buf_load16(rA, vo, (uint32_t)((uint64_t)(kk + u) * p.lda * sizeof(T)));
+      v[u] = matrix_load<NT>(rA, vo, (uint32_t)((uint64_t)(kk + u) * p.lda * sizeof(T)));
       xv[u] = p.x[(int64_t)(kk + u) * p.incx];
     }
 #pragma unroll
@@ -124,7 +138,7 @@ __global__ void __launch_bounds__(256) gemv_n_kernel(GemvParams<T> p) {
     }
   }
   for (; kk < ke; ++kk) {
-    const u32x4 v = buf_load16(rA, vo, (uint32_t)((uint64_t)kk * p.lda * sizeof(T)));
+    const u32x4 v = matrix_load<NT>(rA, vo, (uint32_t)((uint64_t)kk * p.lda * sizeof(T)));
     const T xv = p.x[(int64_t)kk * p.incx];
     const T* a = reinterpret_cast<const T*>(&v);
 #pragma unroll
@@ -149,11 +163,12 @@ __device__ inline T wave_sum(T v) {
 // row when the range is long, of four when it is short.  HBM bound.  Against
 // eight rows of 1 KB per wave with x read from L1, K split only by doubling:
 // FP64 6000 x 4001 43 -> 38 us (5.1 TB/s, matrix not in cache), 2000 x 2500 38
-// -> 12, 16384 x 256 25 -> 12, 8192 x 16384 216 -> 185 (5.8 TB/s), FP32 16000 x
-// 2500 35 -> 34; 16384^2, which fitted that form exactly, 351 -> 361.
+// -> 12, 16384 x 256 25 -> 12, 5000 x 10000 86 -> 75; with the non-temporal hint
+// (matrix_load) 34, 68 and, 16384^2, 351 -> 331 (6.5 TB/s); FP32 16384^2 178 ->
+// 181.
 constexpr int kGemvTWaves = 8;
 constexpr int kGemvTBytes = 32768;  // of x in LDS: four workgroups per CU, whole batches of U chunks
-template <typename T, int RB, int U>
+template <typename T, int RB, int U, bool NT>
 __global__ void __launch_bounds__(64 * kGemvTWaves, 8) gemv_t_kernel(GemvParams<T> p, int rows) {
   constexpr int EPT = 16 / sizeof(T);
   constexpr int CH = 64 * EPT;  // elements of one load of a wave
@@ -173,7 +188,7 @@ __global__ void __launch_bounds__(64 * kGemvTWaves, 8) gemv_t_kernel(GemvParams<
       const uint32_t vo = (uint32_t)(((uint64_t)min(r + b, p.m - 1) * p.lda + lane * EPT) * sizeof(T));
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        v[b][u] = buf_load16(rA, vo, (uint32_t)((uint64_t)(kb + min(c + u, chunks - 1) * CH) * sizeof(T)));
+        v[b][u] = matrix_load<NT>(rA, vo, (uint32_t)((uint64_t)(kb + min(c + u, chunks - 1) * CH) * sizeof(T)));
     }
   };
   T acc[RB][EPT] = {};
@@ -312,12 +327,16 @@ hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, con
   p.W = g.splits > 1 ? static_cast<T*>(workspace) : nullptr;
   p.tickets = trans && g.splits > 1 ? tickets : nullptr;
   dim3 grid((unsigned)g.blocks, (unsigned)g.splits);
-  if (trans && g.batch == 1)
-    hipLaunchKernelGGL((gemv_t_kernel<T, 1, 8>), grid, dim3(64 * kGemvTWaves), 0, s, p, g.rows);
-  else if (trans)
-    hipLaunchKernelGGL((gemv_t_kernel<T, 4, 2>), grid, dim3(64 * kGemvTWaves), 0, s, p, g.rows);
-  else
-    hipLaunchKernelGGL(gemv_n_kernel<T>, grid, dim3(256), 0, s, p);
+  const dim3 threads(trans ? 64 * kGemvTWaves : 256);
+  const bool nt = gemv_streams(trans, bytesA);
+  if (trans) {
+    auto k = g.batch == 1 ? (nt ? gemv_t_kernel<T, 1, 8, true> : gemv_t_kernel<T, 1, 8, false>)
+                          : (nt ? gemv_t_kernel<T, 4, 2, true> : gemv_t_kernel<T, 4, 2, false>);
+    hipLaunchKernelGGL(k, grid, threads, 0, s, p, g.rows);
+  } else {
+    auto k = nt ? gemv_n_kernel<T, true> : gemv_n_kernel<T, false>;
+    hipLaunchKernelGGL(k, grid, threads, 0, s, p);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || g.splits == 1 || p.tickets) return e;
   int64_t rb = (m + 255) / 256;

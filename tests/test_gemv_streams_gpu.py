@@ -53,3 +53,15 @@ def test_gemv_t_exact(gpu, dtype, code, m, n, pad, incx, incy):
         torch.cuda.synchronize()
         g.replay()
         check()
+
+
+@pytest.mark.parametrize("trans,m,n", [(1, 4099, 4097), (1, 300, 60000), (0, 8195, 4099)])
+def test_gemv_past_the_cache_exact(gpu, trans, m, n):
+    """Matrices that are read with the non-temporal hint (from 128 MB for A^T x, 256 MB for Ax)."""
+    g = torch.Generator("cuda").manual_seed(1)
+    a = torch.randint(-3, 4, (n, m), generator=g, device="cuda").double()
+    x, y = (torch.randint(-3, 4, (k,), generator=g, device="cuda").double() for k in ((m, n) if trans else (n, m)))
+    want = 2.0 * (a if trans else a.T) @ x - y
+    E.gemv(E.F64, trans, m, n, 2.0, a.reshape(-1), m, x, 1, -1.0, y, 1)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
