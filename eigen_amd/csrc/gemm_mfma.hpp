@@ -330,9 +330,9 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
   if constexpr (FOLD) {
     static_assert(RS == 2, "folding runs in the two-stage loop");
     fold();
-    epi(total);
+    epi(total, lane, wm, wn);
   } else {
-    epi(acc);
+    epi(acc, lane, wm, wn);
   }
 }
 
@@ -340,11 +340,9 @@ __device__ __forceinline__ void gemm_tile(GemmParams<T> p, int m0, int n0, int k
 // the partial buffer p.W.
 template <typename T, int BM, int BN, int WGM, int WGN, typename Acc>
 __device__ __forceinline__ void tile_store(const GemmParams<T>& p, T alpha, int m0, int n0, int z, bool partial,
-                                           const Acc& acc) {
+                                           const Acc& acc, int lane, int wm, int wn) {
   using F = Mfma<T>;
   constexpr int WTM = BM / WGM, WTN = BN / WGN;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int wm = wid % WGM, wn = wid / WGM;
 #pragma unroll
   for (int i = 0; i < WTM / F::MI; ++i)
 #pragma unroll
@@ -388,7 +386,9 @@ __global__ void __launch_bounds__(64 * WGM * WGN) gemm_mfma_kernel(GemmParams<T>
   const int kend = min(p.K, kbeg + p.k_per_split);
   gemm_tile<T, BM, BN, WGM, WGN, TA, TB, RS, kPlain, false>(
       p, m0, n0, kbeg, kend, smem,
-      [&](const auto& acc) { tile_store<T, BM, BN, WGM, WGN>(p, p.alpha, m0, n0, z, gridDim.y > 1, acc); });
+      [&](const auto& acc, int lane, int wm, int wn) {
+        tile_store<T, BM, BN, WGM, WGN>(p, p.alpha, m0, n0, z, gridDim.y > 1, acc, lane, wm, wn);
+      });
 }
 
 // ---------------------------------------------------------------------------
@@ -511,7 +511,7 @@ __global__ void __launch_bounds__(256, 3) gemm_balanced_kernel(GemmParams<T> p, 
     }
     const int m0 = tm * BM, n0 = tn * BN;
     const int kb = line.begin(r);
-    auto finish = [&](auto& acc) {
+    auto finish = [&](auto& acc, int lane, int wm, int wn) {
       bool store = true;
       if (s0 != 0 || s1 != S) {
         unsigned* ticket = tickets + (int64_t)r * line.cols + c;
@@ -560,7 +560,7 @@ __global__ void __launch_bounds__(256, 3) gemm_balanced_kernel(GemmParams<T> p, 
           }
         }
       }
-      if (store) tile_store<T, BM, BN, 2, 2>(p, MODE == kComplexA ? T(1) : p.alpha, m0, n0, 0, false, acc);
+      if (store) tile_store<T, BM, BN, 2, 2>(p, MODE == kComplexA ? T(1) : p.alpha, m0, n0, 0, false, acc, lane, wm, wn);
     };
     gemm_tile<T, BM, BN, 2, 2, TA, TB, 2, MODE, true>(p, m0, n0, kb + s0 * BK, min(line.end(r), kb + s1 * BK), smem,
                                                       finish);
