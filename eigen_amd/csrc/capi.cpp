@@ -160,15 +160,30 @@ static eh_precision default_sgemm_precision() {
 // stream queue their launch sequences one after another.  Growing replaces
 // the buffer; the old one is freed when its last reference goes, with
 // hipFree, which waits for the device, so work queued with it completes
-// before the memory is released.
+// before the memory is released.  A buffer that a captured call was given
+// stays allocated, since the graph holds its address and may be replayed at
+// any time; its successor is at least twice its size, so that all of a
+// stream's kept buffers together are smaller than the present one.
 struct WorkspaceSlot {
   std::recursive_mutex mu;
   std::shared_ptr<Workspace> buf;
+  std::vector<std::shared_ptr<Workspace>> captured;
 };
 static std::map<std::tuple<int, hipStream_t, std::thread::id>, std::unique_ptr<WorkspaceSlot>> g_ws;
 
 Workspace::~Workspace() {
   if (base) (void)hipFree(base);
+}
+
+// Whether a call on `stream` is recorded into a graph (or cannot be queued
+// there at all, while another stream is captured).
+static bool stream_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return cap != hipStreamCaptureStatusNone;
 }
 
 // Tickets of the balanced products, zero between calls: cleared when the
@@ -221,9 +236,11 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
   lease.lock = std::unique_lock<std::recursive_mutex>(slot->mu);
   if (!slot->buf || slot->buf->bytes < bytes) {
     const size_t have = slot->buf ? slot->buf->bytes : 0;
+    const bool keep = slot->buf && slot->buf->captured;
     auto fresh = std::make_shared<Workspace>();
-    const size_t want = std::max(bytes, std::max(have, (size_t)1 << 20));
-    slot->buf.reset();  // the old buffer goes once no lease refers to it
+    const size_t want = std::max(bytes, std::max(keep ? 2 * have : have, (size_t)1 << 20));
+    if (keep) slot->captured.push_back(std::move(slot->buf));
+    slot->buf.reset();  // any other old buffer goes once no lease refers to it
     e = hipMalloc(&fresh->base, want + kTicketBytes);
     if (e != hipSuccess) {
       fresh->base = nullptr;
@@ -234,6 +251,7 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
     slot->buf = std::move(fresh);
   }
   lease.buf = slot->buf;
+  lease.buf->captured |= stream_capturing(stream);
   *ptr = lease.buf->ptr;
   *out = std::move(lease);
   return EH_SUCCESS;
@@ -560,13 +578,7 @@ static eh_status launch_product(bool ta, bool tb, int64_t m, int64_t n, int64_t 
 // stream's workspace.  (A plain product then keeps its configuration, run_gemm
 // below.)
 static bool balanced_workspace_allowed(hipStream_t stream) {
-  if (fixed_scratch_active()) return true;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return cap == hipStreamCaptureStatusNone;
+  return fixed_scratch_active() || !stream_capturing(stream);
 }
 
 // Workgroups the balanced kernel runs: it fits three to a CU, and short runs

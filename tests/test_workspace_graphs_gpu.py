@@ -1,0 +1,51 @@
+"""Graphs that hold a stream's workspace, and the workspace's growth around
+them: integer operands, so every result is exact."""
+import numpy as np
+import pytest
+import torch
+
+import eigen_amd as E
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(m, n, k, seed):
+    A, B = O.fill((m, k), np.float64, seed, O.INT, -3, 3), O.fill((k, n), np.float64, seed + 1, O.INT, -3, 3)
+    dev = [torch.from_numpy(x.reshape(-1, order="F").copy()).cuda() for x in (A, B)]
+    return dev, torch.from_numpy((A @ B).reshape(-1, order="F").copy()).cuda()
+
+
+def product(m, n, k, ab, c, stream):
+    E.gemm(E.F64, 0, 0, m, n, k, 1.0, ab[0], m, ab[1], k, 0.0, c, m, prec=E.PREC_PLAIN, stream=stream.cuda_stream)
+
+
+def test_graph_outlives_growth(gpu):
+    """A graph with a split-K product keeps its partial sums' buffer when later
+    calls on its stream need a larger one, twice."""
+    m, n, k = 130, 130, 20000
+    assert E.config_info(E.plan(E.F64, 0, 0, m, n, k))[2] > 1
+    ab, want = operands(m, n, k, 1)
+    c = torch.zeros_like(want)
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        product(m, n, k, ab, c, s)
+        torch.cuda.synchronize()
+        g.capture_begin()
+        product(m, n, k, ab, c, s)
+        g.capture_end()
+    for big in ((1000, 777, 1203), (1024, 1100, 9000)):
+        bab, bwant = operands(*big, 5)
+        bc = torch.zeros_like(bwant)
+        with torch.cuda.stream(s):
+            product(*big, bab, bc, s)
+        torch.cuda.synchronize()
+        assert torch.equal(bc, bwant)
+        hold = torch.full((1 << 24,), float("nan"), dtype=torch.float64, device="cuda")  # takes freed memory
+        for _ in range(2):
+            c.zero_()
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, want)
+        assert torch.isnan(hold).all()
