@@ -236,6 +236,16 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
   lease.lock = std::unique_lock<std::recursive_mutex>(slot->mu);
   if (!slot->buf || slot->buf->bytes < bytes) {
     const size_t have = slot->buf ? slot->buf->bytes : 0;
+    // hipMalloc and hipFree end every capture in progress, on any stream,
+    // unless the calling thread's mode says that it does not mean them to
+    struct RelaxedCapture {
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      const bool set;
+      explicit RelaxedCapture(bool on) : set(on && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+      ~RelaxedCapture() {
+        if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+      }
+    } relaxed(!stream_capturing(stream));
     const bool keep = slot->buf && slot->buf->captured;
     auto fresh = std::make_shared<Workspace>();
     const size_t want = std::max(bytes, std::max(keep ? 2 * have : have, (size_t)1 << 20));

@@ -49,3 +49,30 @@ def test_graph_outlives_growth(gpu):
             torch.cuda.synchronize()
             assert torch.equal(c, want)
         assert torch.isnan(hold).all()
+
+
+@pytest.mark.parametrize("before", [False, True])
+def test_eager_call_beside_a_capture(gpu, before):
+    """A product on one stream that needs that stream's first workspace, or a
+    larger one, leaves the capture of another stream intact."""
+    first = (1000, 777, 1203)
+    ab, want = operands(96, 80, 112, 1)
+    fab, fwant = operands(*first, 3)
+    c, fc = torch.zeros_like(want), torch.zeros_like(fwant)
+    s, t, g = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    if before:
+        product(130, 130, 2000, *operands(130, 130, 2000, 7), t)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        g.capture_begin()
+        product(96, 80, 112, ab, c, s)
+        product(*first, fab, fc, t)
+        g.capture_end()
+    torch.cuda.synchronize()
+    assert torch.equal(fc, fwant)
+    for _ in range(2):
+        c.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want)
