@@ -23,6 +23,8 @@
 // rows past m only feed outputs that are never stored.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -168,78 +170,95 @@ __device__ inline T wave_sum(T v) {
 // 181.
 constexpr int kGemvTWaves = 8;
 constexpr int kGemvTBytes = 32768;  // of x in LDS: four workgroups per CU, whole batches of U chunks
-template <typename T, int RB, int U, bool NT>
+// PARTS: the split is longer than one LDS part; the parts follow one another,
+// the sums of the workgroup's rows so far in LDS (16M FP64 elements by one row:
+// 79 us, 172 with one split per part, whose 1954 sums one thread added).
+template <typename T, int RB, int U, bool NT, bool PARTS>
 __global__ void __launch_bounds__(64 * kGemvTWaves, 8) gemv_t_kernel(GemvParams<T> p, int rows) {
   constexpr int EPT = 16 / sizeof(T);
   constexpr int CH = 64 * EPT;  // elements of one load of a wave
-  __shared__ __attribute__((aligned(16))) T xs[kGemvTBytes / sizeof(T)];
+  constexpr int PART = kGemvTBytes / sizeof(T);
+  __shared__ __attribute__((aligned(16))) T xs[PART];
+  __shared__ T sums[PARTS ? 2 * kGemvTWaves * RB : 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int z = blockIdx.y;
-  const int kb = z * p.k_per_split, len = min(p.k - kb, p.k_per_split);
-  const int chunks = (len + CH - 1) / CH;
-  for (int i = threadIdx.x; i < (chunks + U - 1) / U * U * CH; i += 64 * kGemvTWaves)
-    xs[i] = i < len ? p.x[(int64_t)(kb + i) * p.incx] : T(0);
-  __syncthreads();
+  const int kz = z * p.k_per_split, ke = min(p.k, kz + p.k_per_split);
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, p.bytesA);
   const int i0 = blockIdx.x * rows, i1 = min(p.m, i0 + rows);
-  auto load = [&](int r, int c, u32x4(&v)[RB][U]) {
-#pragma unroll
-    for (int b = 0; b < RB; ++b) {
-      const uint32_t vo = (uint32_t)(((uint64_t)min(r + b, p.m - 1) * p.lda + lane * EPT) * sizeof(T));
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        v[b][u] = matrix_load<NT>(rA, vo, (uint32_t)((uint64_t)(kb + min(c + u, chunks - 1) * CH) * sizeof(T)));
-    }
-  };
-  T acc[RB][EPT] = {};
-  // every wave starts its rows at another batch of the range: rows a power of
-  // two apart would otherwise all be read at one memory channel's addresses
-  const int batches = (chunks + U - 1) / U;
-  const int c0 = (int)((blockIdx.x * kGemvTWaves + wave) % batches) * U;
-  int r = i0 + wave * RB, c = c0;
-  while (r < i1) {
-    u32x4 v[RB][U];
-    load(r, c, v);
-    const int cn = c + U >= chunks ? 0 : c + U;
-    const bool row_ends = cn == c0;
-    const int rn = row_ends ? r + kGemvTWaves * RB : r;
-    if ((c + U) * CH > len) {
-      // elements past the range (the next row's data, the next split's, a
-      // repeated chunk) meet x = 0 only if they are finite; select them away
-#pragma unroll
-      for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int e = 0; e < EPT; ++e) {
-            T* a = reinterpret_cast<T*>(&v[b][u]);
-            a[e] = (c + u) * CH + lane * EPT + e < len ? a[e] : T(0);
-          }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const u32x4 xv = *reinterpret_cast<const u32x4*>(&xs[(c + u) * CH + lane * EPT]);
-#pragma unroll
-      for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int e = 0; e < EPT; ++e)
-          acc[b][e] = fma_t(reinterpret_cast<const T*>(&v[b][u])[e], reinterpret_cast<const T*>(&xv)[e], acc[b][e]);
-    }
-    if (row_ends) {
+  int kb = kz;
+  do {
+    const int len = PARTS ? min(ke - kb, PART) : ke - kb;
+    const int chunks = (len + CH - 1) / CH;
+    if (PARTS && kb != kz) __syncthreads();  // xs is free again
+    for (int i = threadIdx.x; i < (chunks + U - 1) / U * U * CH; i += 64 * kGemvTWaves)
+      xs[i] = i < len ? p.x[(int64_t)(kb + i) * p.incx] : T(0);
+    __syncthreads();
+    auto load = [&](int r, int c, u32x4(&v)[RB][U]) {
 #pragma unroll
       for (int b = 0; b < RB; ++b) {
-        T s = acc[b][0];
+        const uint32_t vo = (uint32_t)(((uint64_t)min(r + b, p.m - 1) * p.lda + lane * EPT) * sizeof(T));
 #pragma unroll
-        for (int e = 1; e < EPT; ++e) s += acc[b][e];
-        s = wave_sum(s);
-        if (lane == 0 && r + b < i1) gemv_store(p, r + b, s, z);
-#pragma unroll
-        for (int e = 0; e < EPT; ++e) acc[b][e] = T(0);
+        for (int u = 0; u < U; ++u)
+          v[b][u] = matrix_load<NT>(rA, vo, (uint32_t)((uint64_t)(kb + min(c + u, chunks - 1) * CH) * sizeof(T)));
       }
+    };
+    T acc[RB][EPT] = {};
+    // every wave starts its rows at another batch of the range: rows a power of
+    // two apart would otherwise all be read at one memory channel's addresses
+    const int batches = (chunks + U - 1) / U;
+    const int c0 = (int)((blockIdx.x * kGemvTWaves + wave) % batches) * U;
+    int r = i0 + wave * RB, c = c0;
+    while (r < i1) {
+      u32x4 v[RB][U];
+      load(r, c, v);
+      const int cn = c + U >= chunks ? 0 : c + U;
+      const bool row_ends = cn == c0;
+      const int rn = row_ends ? r + kGemvTWaves * RB : r;
+      if ((c + U) * CH > len) {
+        // elements past the range (the next row's data, the next split's, a
+        // repeated chunk) meet x = 0 only if they are finite; select them away
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < EPT; ++e) {
+              T* a = reinterpret_cast<T*>(&v[b][u]);
+              a[e] = (c + u) * CH + lane * EPT + e < len ? a[e] : T(0);
+            }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const u32x4 xv = *reinterpret_cast<const u32x4*>(&xs[(c + u) * CH + lane * EPT]);
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+          for (int e = 0; e < EPT; ++e)
+            acc[b][e] = fma_t(reinterpret_cast<const T*>(&v[b][u])[e], reinterpret_cast<const T*>(&xv)[e], acc[b][e]);
+      }
+      if (row_ends) {
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+          T s = acc[b][0];
+#pragma unroll
+          for (int e = 1; e < EPT; ++e) s += acc[b][e];
+          s = wave_sum(s);
+          if (lane == 0 && r + b < i1) {
+            if (PARTS && kb != kz) s += sums[r + b - i0];  // the wave's own: its rows are the same in every part
+            if (PARTS && kb + len < ke)
+              sums[r + b - i0] = s;
+            else
+              gemv_store(p, r + b, s, z);
+          }
+#pragma unroll
+          for (int e = 0; e < EPT; ++e) acc[b][e] = T(0);
+        }
+      }
+      r = rn;
+      c = cn;
     }
-    r = rn;
-    c = cn;
-  }
+    kb += len;
+  } while (PARTS && kb < ke);
   gemv_finish(p, i0, i1);
 }
 
@@ -250,18 +269,20 @@ __global__ void __launch_bounds__(256) gemv_reduce_kernel(GemvParams<T> p, int s
 
 // Grid of a matrix-vector product: row blocks, and splits of K.
 //
-// Aᵀx: splits whose part of x fits in LDS, in whole batches of loads; among
-// them, and one or two rows (or groups of rows) per wave, the plan whose rounds
+// Aᵀx: splits whose part of x fits in LDS (past kGemvTSplits of them, several
+// parts to a split: one thread adds a row's partial sums, sixteen loads at a
+// time), in whole batches of loads; among them, and one or two rows (or groups of rows) per wave, the plan whose rounds
 // of resident workgroups (four per CU) stream the fewest bytes, x's part
 // counted as one row and a workgroup's start as 16 KB.  More rows per workgroup
 // leave the last round uneven (16384^2 FP64: 361, 363, 368 us with 16, 32, 64).
+constexpr int kGemvTSplits = 256;
 static GemvPlan gemv_t_plan(int m, int k, int es) {
   constexpr int kGroups = 1024;
   const int chunk = 64 * 16 / es;
   GemvPlan best{};
   double best_cost = 0;
-  const int smin = (int)(((int64_t)k * es + kGemvTBytes - 1) / kGemvTBytes);
-  for (int s = smin; s == smin || (s < smin + 16 && (int64_t)k * es >= (int64_t)s * 4096); ++s) {
+  const int smin = (int)std::min<int64_t>(kGemvTSplits, ((int64_t)k * es + kGemvTBytes - 1) / kGemvTBytes);
+  for (int s = smin; s == smin || (s < smin + 16 && s <= kGemvTSplits && (int64_t)k * es >= (int64_t)s * 4096); ++s) {
     int64_t per = ((int64_t)k + s - 1) / s;
     GemvPlan g{};
     g.batch = per >= 6 * chunk ? 1 : 4;
@@ -330,8 +351,10 @@ hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, con
   const dim3 threads(trans ? 64 * kGemvTWaves : 256);
   const bool nt = gemv_streams(trans, bytesA);
   if (trans) {
-    auto k = g.batch == 1 ? (nt ? gemv_t_kernel<T, 1, 8, true> : gemv_t_kernel<T, 1, 8, false>)
-                          : (nt ? gemv_t_kernel<T, 4, 2, true> : gemv_t_kernel<T, 4, 2, false>);
+    const bool parts = (int64_t)g.per * (int)sizeof(T) > kGemvTBytes;
+    auto k = parts          ? (nt ? gemv_t_kernel<T, 1, 8, true, true> : gemv_t_kernel<T, 1, 8, false, true>)
+             : g.batch == 1 ? (nt ? gemv_t_kernel<T, 1, 8, true, false> : gemv_t_kernel<T, 1, 8, false, false>)
+                            : (nt ? gemv_t_kernel<T, 4, 2, true, false> : gemv_t_kernel<T, 4, 2, false, false>);
     hipLaunchKernelGGL(k, grid, threads, 0, s, p, g.rows);
   } else {
     auto k = nt ? gemv_n_kernel<T, true> : gemv_n_kernel<T, false>;

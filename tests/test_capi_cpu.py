@@ -344,6 +344,18 @@ def test_triangular_tile_enumeration(tmp_path):
     assert out.returncode == 0 and "ALL PASSED" in out.stdout, out.stdout
 
 
+def test_matrix_vector_plans(tmp_path):
+    """gemv_plan over every size one launch takes: at most 256 splits of K, and
+    partial sums that fit the allocation-free entry's scratch."""
+    exe = tmp_path / "gemv_plan_check"
+    src = os.path.join(ROOT, "tests", "gemv_plan_check.cpp")
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "-O2", "-std=c++17", "-o", str(exe), src, "-L", E.LIBDIR, "-leigen_amd",
+                        "-Wl,-rpath," + os.path.abspath(E.LIBDIR)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0 and "ALL PASSED" in out.stdout, out.stdout
+
+
 def test_batched_strided_argument_checks():
     L = E.lib()
     one = C.c_double(1.0)

@@ -65,3 +65,27 @@ def test_gemv_past_the_cache_exact(gpu, trans, m, n):
     E.gemv(E.F64, trans, m, n, 2.0, a.reshape(-1), m, x, 1, -1.0, y, 1)
     torch.cuda.synchronize()
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("m,n,incx", [(2 ** 21 + 5, 1, 1), (2 ** 21 - 7, 3, 2), (40_000_003, 1, 1), (3_000_001, 4, 1),
+                                      (4_200_000, 17, 1)])
+def test_long_inner_products_exact(gpu, dtype, m, n, incx):
+    """A^T x past 256 parts of x in LDS: several parts to a split, the sums of a
+    block's rows kept between them; every sum is below 2^24."""
+    g = torch.Generator("cuda").manual_seed(m)
+    a = torch.zeros(n, m, dtype=dtype, device="cuda")
+    x = torch.full(((m - 1) * incx + 1,), float("nan"), dtype=dtype, device="cuda")
+    x[::incx] = torch.randint(-2, 3, (m,), generator=g, device="cuda").to(dtype)
+    for j in range(n):
+        a[j] = torch.randint(0, 2, (m,), generator=g, device="cuda").to(dtype)
+    a[:, -1] = 1
+    y0 = torch.arange(n, dtype=dtype, device="cuda")
+    want = [2 * int((a[j].long() * x[::incx].long()).sum()) - j for j in range(n)]
+    assert max(map(abs, want)) < 1 << 23
+    code = E.F32 if dtype == torch.float32 else E.F64
+    for _ in range(2):
+        y = y0.clone()
+        E.gemv(code, 1, m, n, 2.0, a.reshape(-1), m, x, incx, -1.0, y, 1)
+        torch.cuda.synchronize()
+        assert y.long().tolist() == want
