@@ -2,7 +2,8 @@
 // launch takes (extent below 4 GB, both types and directions): the splits
 // cover k, are at most 256 (a grid's y dimension ends at 65,536, and one
 // thread adds a row's partial sums), and their partial sums fit the
-// allocation-free entry's scratch.  Built and run by tests/test_capi_cpu.py.
+// allocation-free entry's scratch; rows of A^T x that one load of a wave holds
+// are not split.  Built and run by tests/test_capi_cpu.py.
 #include <cmath>
 #include <cstdio>
 #include <random>
@@ -24,6 +25,11 @@ int main() {
         if (i == 2) m = 4, k = 100000000;
         const eh::GemvPlan g = eh::gemv_plan(trans, (int)m, (int)k, es);
         const size_t ws = eh::gemv_workspace_bytes(g, (int)m, es);
+        if (trans && k * es <= 1024 && (g.splits != 1 || g.batch != 8 || (int64_t)g.blocks * g.rows < m)) {
+          std::printf("FAIL short rows es=%d m=%lld k=%lld: %d splits, batch %d\n", es, (long long)m, (long long)k, g.splits,
+                      g.batch);
+          return 1;
+        }
         if (g.blocks < 1 || g.splits < 1 || g.splits > 256 || (int64_t)g.per * g.splits < k ||
             (int64_t)g.per * (g.splits - 1) >= k || ws > EH_NOALLOC_SCRATCH_BYTES) {
           std::printf("FAIL trans=%d es=%d m=%lld k=%lld: %d splits of %d, %d blocks, %zu bytes\n", trans, es, (long long)m,

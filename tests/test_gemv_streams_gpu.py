@@ -89,3 +89,24 @@ def test_long_inner_products_exact(gpu, dtype, m, n, incx):
         E.gemv(code, 1, m, n, 2.0, a.reshape(-1), m, x, incx, -1.0, y, 1)
         torch.cuda.synchronize()
         assert y.long().tolist() == want
+
+
+@pytest.mark.parametrize("dtype,code", [(np.float32, E.F32), (np.float64, E.F64)])
+@pytest.mark.parametrize("m", [1, 3, 64, 127, 128, 129, 255, 256, 257])
+@pytest.mark.parametrize("n,pad,incx,incy", [(1, 0, 1, 1), (31, 1, 2, 1), (33, 3, -1, 2), (5000, 0, 1, -1)])
+def test_gemv_t_short_rows_exact(gpu, dtype, code, m, n, pad, incx, incy):
+    """Rows around one 1 KB load of a wave (128 FP64, 256 FP32 elements): each is
+    followed by NaN, or by the next row, where it ends."""
+    A = O.fill((m + pad, n), dtype, 1, O.INT, -3, 3)
+    A[m:] = np.nan
+    x, y = O.fill((m, 1), dtype, 2, O.INT, -3, 3)[:, 0], O.fill((n, 1), dtype, 3, O.INT, -3, 3)[:, 0]
+    want = 2.0 * (A[:m].astype(np.float64).T @ x) - y
+    dx = np.full((m - 1) * abs(incx) + 1, np.nan, dtype)
+    dx[::abs(incx)] = x if incx > 0 else x[::-1]
+    dy = np.full((n - 1) * abs(incy) + 1, np.nan, dtype)
+    dy[::abs(incy)] = y if incy > 0 else y[::-1]
+    a, dx, dy = (torch.from_numpy(v).cuda() for v in (A.reshape(-1, order="F").copy(), dx, dy))
+    E.gemv(code, 1, m, n, 2.0, a, m + pad, dx, incx, -1.0, dy, incy)
+    torch.cuda.synchronize()
+    got = dy.cpu().numpy()[::abs(incy)]
+    assert np.array_equal((got if incy > 0 else got[::-1]).astype(np.float64), want)
