@@ -354,7 +354,8 @@ static GemvPlan gemv_t_plan(int m, int k, int es) {
 
 // Ax: about 256 workgroups' worth of streaming, one long-running workgroup per
 // CU: each then streams long runs of its columns, where 2048 shorter workgroups
-// measured 10-20% slower.  Splits of 32 columns while they are few (FP64 12000 x
+// measured 10-20% slower.  Below 128 columns no split, whose second launch takes
+// longer than the columns (64^2: 10.3 us, 7.5 without).  Splits of 32 columns while they are few (FP64 12000 x
 // 300: 15.1 -> 11.1 us, 1000^2 11.5 -> 10.3), of 64 after that: adding up many
 // takes longer than they save (FP32 300 x 12000: 14.4 against 16.3 us).
 GemvPlan gemv_plan(bool trans, int m, int k, int es) {
@@ -363,7 +364,7 @@ GemvPlan gemv_plan(bool trans, int m, int k, int es) {
   GemvPlan g{};
   g.blocks = (m + 256 * ept - 1) / (256 * ept);
   int s = 1;
-  while ((int64_t)g.blocks * s < 256 && k / (2 * s) >= (s <= 16 ? 32 : 64) && s < 256) s *= 2;
+  while ((int64_t)g.blocks * s < 256 && k / (2 * s) >= (k >= 128 && s <= 16 ? 32 : 64) && s < 256) s *= 2;
   int64_t per = ((int64_t)k + s - 1) / s;
   per = (per + chunk - 1) / chunk * chunk;
   g.per = (int)per;

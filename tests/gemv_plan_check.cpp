@@ -3,7 +3,7 @@
 // cover k, are at most 256 (a grid's y dimension ends at 65,536, and one
 // thread adds a row's partial sums), and their partial sums fit the
 // allocation-free entry's scratch; rows of A^T x that one load of a wave holds
-// are not split.  Built and run by tests/test_capi_cpu.py.
+// are not split, nor is Ax below 128 columns.  Built and run by tests/test_capi_cpu.py.
 #include <cmath>
 #include <cstdio>
 #include <random>
@@ -28,6 +28,10 @@ int main() {
         if (trans && k * es <= 1024 && (g.splits != 1 || g.batch != 8 || (int64_t)g.blocks * g.rows < m)) {
           std::printf("FAIL short rows es=%d m=%lld k=%lld: %d splits, batch %d\n", es, (long long)m, (long long)k, g.splits,
                       g.batch);
+          return 1;
+        }
+        if (!trans && k < 128 && g.splits != 1) {
+          std::printf("FAIL few columns es=%d m=%lld k=%lld: %d splits\n", es, (long long)m, (long long)k, g.splits);
           return 1;
         }
         if (g.blocks < 1 || g.splits < 1 || g.splits > 256 || (int64_t)g.per * g.splits < k ||
