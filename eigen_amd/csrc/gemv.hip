@@ -112,7 +112,12 @@ template <bool NT>
 __device__ inline u32x4 matrix_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   return NT ? buf_load16_stream(r, voff, soff) : buf_load16(r, voff, soff);
 }
-static bool gemv_streams(bool trans, uint32_t bytes) { return bytes >= (trans ? 128u : 256u) << 20; }
+// Short columns of Ax share lines with their neighbours, which the hint drops
+// between the two reads: FP64 250 x 400,000 155 us without, 173 with it, 500 x
+// 200,000 143 and 126; FP32 100 x 1,000,000 339 and 359, 500 x 200,000 101 and 96.
+bool gemv_streams(bool trans, int m, uint32_t bytes) {
+  return bytes >= (trans ? 128u : 256u) << 20 && (trans || m >= 384);
+}
 
 // k unroll of gemv_n_kernel (loads in flight per thread): 16 for FP64
 // (16384^2: 370 -> 362 us), 8 for FP32 (16 measured 2% slower).
@@ -397,7 +402,7 @@ hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, con
   p.W = g.splits > 1 ? static_cast<T*>(workspace) : nullptr;
   p.tickets = trans && g.splits > 1 ? tickets : nullptr;
   dim3 grid((unsigned)g.blocks, (unsigned)g.splits);
-  const bool nt = gemv_streams(trans, bytesA);
+  const bool nt = gemv_streams(trans, m, bytesA);
   const bool short_rows = trans && g.batch == kGemvShortRows;
   const dim3 threads(trans && !short_rows ? 64 * kGemvTWaves : 256);
   if (short_rows) {

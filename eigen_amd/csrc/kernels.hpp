@@ -74,6 +74,8 @@ struct GemvPlan {
 // row block adds its partial sums and no second launch follows.
 GemvPlan gemv_plan(bool trans, int m, int k, int es);
 size_t gemv_workspace_bytes(const GemvPlan& g, int m, int es);
+// Whether a matrix of `bytes` is read with the non-temporal hint.
+bool gemv_streams(bool trans, int m, uint32_t bytes);
 template <typename T>
 hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, const T* A, int64_t lda,
                        uint32_t bytesA, const T* x, int64_t incx, T beta, T* y, int64_t incy, void* workspace,

@@ -42,6 +42,13 @@ int main() {
         }
         ++checked;
       }
+  // short columns share cache lines: never read with the non-temporal hint
+  for (int m : {1, 50, 100, 250, 500, 4096}) {
+    if (eh::gemv_streams(false, m, 1u << 30) != (m >= 500) || eh::gemv_streams(false, m, 1u << 27)) {
+      std::printf("FAIL hint for Ax of %d rows\n", m);
+      return 1;
+    }
+  }
   std::printf("ALL PASSED (%lld)\n", (long long)checked);
   return 0;
 }
