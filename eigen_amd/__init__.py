@@ -203,6 +203,7 @@ def _declare_extra(L) -> None:
         "eh_tuner_clear": (i32, []),
         "eh_num_packed_configs": (i32, [i32]),
         "eh_packed_config_info": (i32, [i32, i32, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
+        "eh_plan_kernel": (i32, [i32, i32, i32, i64, i64, i64, C.POINTER(i32)]),
         "eh_plan_packed": (i32, [i32, i32, i32, i64, i64, i64, C.POINTER(i32)]),
         "eh_time_config_packed": (i32, [i32, i32, i32, i64, i64, i64, vp, vp, vp, i32, i32, C.POINTER(f32)]),
         "eh_tuner_record_packed": (i32, [i32, i32, i32, i64, i64, i64, i32]),
@@ -451,6 +452,16 @@ def config_info(config: int):
 def plan(dtype: int, opa: int, opb: int, m: int, n: int, k: int) -> int:
     c = C.c_int()
     check(lib().eh_plan(dtype, opa, opb, m, n, k, C.byref(c)), "eh_plan")
+    return c.value
+
+
+KERNEL_CONFIG, KERNEL_SMALL, KERNEL_BALANCED, KERNEL_VECTOR = 0, 1, 2, 3
+
+
+def plan_kernel(dtype: int, opa: int, opb: int, m: int, n: int, k: int) -> int:
+    """Kernel a plain-precision eh_gemm runs for this shape on dense operands (eh_product_kernel)."""
+    c = C.c_int()
+    check(lib().eh_plan_kernel(dtype, opa, opb, m, n, k, C.byref(c)), "eh_plan_kernel")
     return c.value
 
 

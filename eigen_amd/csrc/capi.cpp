@@ -774,6 +774,31 @@ static bool small_product(int64_t m, int64_t n, int64_t k) {
   return tiles <= 2 * kCUs && (k <= 512 || (k <= 1024 && tiles >= kCUs / 4));
 }
 
+// Whether products leave the planner's configurations for the small and
+// balanced kernels: a caller who chose another planner, or a network of its own,
+// gets what that chooses.
+static bool own_rules() { return tune_mode() == EH_TUNE_MLP && !mlp_installed(); }
+
+// Kernel of a plain-precision product, and its configuration unless small.
+template <typename T>
+static eh_status product_kernel(int opa, int opb, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                                eh_product_kernel* kernel, int* config) {
+  constexpr bool f64 = std::is_same<T, double>::value;
+  const bool ta = opa != EH_OP_N, tb = opb != EH_OP_N;
+  const bool own = own_rules() && operand_fits<T>(ta, m, k, lda) && operand_fits<T>(!tb, n, k, ldb);
+  if (own && small_product(m, n, k)) {
+    const GemmParams<T> p = product_params<T>(ta, tb, m, n, k, T(0), nullptr, lda, nullptr, ldb, T(0), nullptr, m);
+    if (std::max(p.bytesA, p.bytesB) < 0x80000000u) {
+      *kernel = EH_KERNEL_SMALL;
+      return EH_SUCCESS;
+    }
+  }
+  eh_status st = plan_config(f64 ? EH_F64 : EH_F32, opa, opb, m, n, k, config);
+  if (st != EH_SUCCESS) return st;
+  *kernel = own && balanced_pays(f64, m, n, k, *config) ? EH_KERNEL_BALANCED : EH_KERNEL_CONFIG;
+  return EH_SUCCESS;
+}
+
 template <typename T>
 static eh_status run_gemm(int opa, int opb, int64_t m, int64_t n, int64_t k, T alpha, const T* A, int64_t lda,
                           const T* B, int64_t ldb, T beta, T* C, int64_t ldc, eh_precision prec, int config,
@@ -806,27 +831,21 @@ static eh_status run_gemm(int opa, int opb, int64_t m, int64_t n, int64_t k, T a
     if (vector_product<T>(opa, opb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, stream, &st)) return st;
   }
   if (!split_prec && config < 0) {
-    const bool own_rules = tune_mode() == EH_TUNE_MLP && !mlp_installed() && operand_fits<T>(ta, m, k, lda) &&
-                           operand_fits<T>(!tb, n, k, ldb);
-    if (own_rules && small_product(m, n, k)) {
-      const GemmParams<T> p = product_params<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-      if (std::max(p.bytesA, p.bytesB) < 0x80000000u) {
-        KernelTimer t(EH_KC_PRODUCT, stream);
-        e = launch_gemm_small<T>(p, ta, tb, stream);
-        return e == hipSuccess ? EH_SUCCESS : hip_fail(e, "small product launch");
-      }
-    }
-    eh_status st = plan_config(std::is_same<T, float>::value ? EH_F32 : EH_F64, opa, opb, m, n, k, &config);
+    eh_product_kernel kernel;
+    eh_status st = product_kernel<T>(opa, opb, m, n, k, lda, ldb, &kernel, &config);
     if (st != EH_SUCCESS) return st;
-    if (own_rules) {
-      if (balanced_pays(std::is_same<T, double>::value, m, n, k, config) && balanced_workspace_allowed(stream)) {
-        // the workspace grows to what `config` needs too: a caller may run a
-        // product once before it captures it
-        int t = 0, splits = 1;
-        config_decode(config, &t, &splits);
-        return launch_balanced<T>(product_params<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc), kPlain, ta,
-                                  tb, stream, splits > 1 ? (size_t)splits * m * n * sizeof(T) : 0);
-      }
+    const GemmParams<T> p = product_params<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+    if (kernel == EH_KERNEL_SMALL) {
+      KernelTimer t(EH_KC_PRODUCT, stream);
+      e = launch_gemm_small<T>(p, ta, tb, stream);
+      return e == hipSuccess ? EH_SUCCESS : hip_fail(e, "small product launch");
+    }
+    if (kernel == EH_KERNEL_BALANCED && balanced_workspace_allowed(stream)) {
+      // the workspace grows to what `config` needs too: a caller may run a
+      // product once before it captures it
+      int t = 0, splits = 1;
+      config_decode(config, &t, &splits);
+      return launch_balanced<T>(p, kPlain, ta, tb, stream, splits > 1 ? (size_t)splits * m * n * sizeof(T) : 0);
     }
   }
   return launch_product<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, split_prec, terms, config, stream);
@@ -1108,6 +1127,24 @@ eh_status eh_plan(eh_dtype dtype, eh_op opa, eh_op opb, int64_t m, int64_t n, in
   if (dtype != EH_F32 && dtype != EH_F64) return fail(EH_ERR_INVALID, "bad dtype");
   if (m < 0 || n < 0 || k < 0) return fail(EH_ERR_INVALID, "m, n, k must be >= 0");
   return plan_config(dtype, opa, opb, m, n, k, config);
+}
+
+eh_status eh_plan_kernel(eh_dtype dtype, eh_op opa, eh_op opb, int64_t m, int64_t n, int64_t k,
+                         eh_product_kernel* kernel) {
+  if (!kernel) return fail(EH_ERR_INVALID, "kernel is NULL");
+  if (dtype != EH_F32 && dtype != EH_F64) return fail(EH_ERR_INVALID, "bad dtype");
+  if (!valid_op(opa) || !valid_op(opb)) return fail(EH_ERR_INVALID, "opa and opb must be N, T or C");
+  if (m < 1 || n < 1 || k < 1) return fail(EH_ERR_INVALID, "m, n, k must be >= 1");
+  if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return fail(EH_ERR_UNSUPPORTED, "m, n, k must fit int32");
+  const int64_t lda = opa == EH_OP_N ? m : k, ldb = opb == EH_OP_N ? k : n;
+  const uint64_t es = dtype == EH_F64 ? sizeof(double) : sizeof(float);
+  if ((m == 1 || n == 1) && ((uint64_t)std::max(m, n) * (uint64_t)k + 64) * es < kMaxExtent) {
+    *kernel = EH_KERNEL_VECTOR;
+    return EH_SUCCESS;
+  }
+  int config = -1;
+  return dtype == EH_F64 ? product_kernel<double>(opa, opb, m, n, k, lda, ldb, kernel, &config)
+                         : product_kernel<float>(opa, opb, m, n, k, lda, ldb, kernel, &config);
 }
 
 eh_status eh_set_tune_mode(eh_tune_mode mode) {

@@ -38,7 +38,7 @@
  *       and the level-3 kernels they run (GeneralMatrixMatrixTriangular.h,
  *       SelfadjointMatrixMatrix.h, TriangularMatrixMatrix.h,
  *       TriangularSolverMatrix.h), on the same MFMA product kernels.
- *   eh_plan / eh_set_tune_mode
+ *   eh_plan / eh_plan_kernel / eh_set_tune_mode
  *       computeProductBlockingSizes + evaluateProductBlockingSizesHeuristic
  *       (GeneralBlockPanelKernel.h:201-452): the blocking choice, here a
  *       tile/split-K configuration picked by a heuristic, a trained MLP or an
@@ -371,8 +371,23 @@ eh_status eh_gemmtr_complex(eh_dtype dtype, eh_uplo uplo, eh_op opa, eh_op opb, 
 int eh_num_configs(void);
 /* Tile (tile_m x tile_n) and split-K factor of configuration `config`. */
 eh_status eh_config_info(int config, int* tile_m, int* tile_n, int* split_k);
-/* Configuration the planner would use for this shape (synchronous). */
+/* Configuration the planner would use for this shape (synchronous).  Under
+ * EH_TUNE_MLP with the compiled-in network, eh_gemm leaves it for another kernel
+ * on some shapes (eh_plan_kernel); the configurations stay what eh_gemm_config,
+ * EH_TUNE_HEURISTIC, EH_TUNE_TABLE and an installed network choose among. */
 eh_status eh_plan(eh_dtype dtype, eh_op opa, eh_op opb, int64_t m, int64_t n, int64_t k, int* config);
+/* Kernel that eh_gemm in plain precision runs for this shape on dense operands
+ * (m, n, k >= 1).  A call that is captured into a graph runs eh_plan's
+ * configuration in place of EH_KERNEL_BALANCED, whose workgroups meet in the
+ * stream's workspace. */
+typedef enum eh_product_kernel {
+  EH_KERNEL_CONFIG = 0,   /* eh_plan's configuration */
+  EH_KERNEL_SMALL = 1,    /* 32x32 tiles, a workgroup's waves share k */
+  EH_KERNEL_BALANCED = 2, /* 64x64 tiles, cut evenly between the workgroups the chip holds */
+  EH_KERNEL_VECTOR = 3    /* m or n is 1: matrix-vector kernels */
+} eh_product_kernel;
+eh_status eh_plan_kernel(eh_dtype dtype, eh_op opa, eh_op opb, int64_t m, int64_t n, int64_t k,
+                         eh_product_kernel* kernel);
 eh_status eh_set_tune_mode(eh_tune_mode mode);
 eh_tune_mode eh_get_tune_mode(void);
 eh_status eh_set_sgemm_precision(eh_precision prec);
