@@ -642,26 +642,48 @@ static bool many_large_tiles(bool f64, int64_t m, int64_t n) {
   return ((m + 127) / 128) * ((n + 127) / 128) >= (f64 ? 2 : 1) * kCUs;
 }
 
-// Whether a plain product leaves configuration `config` for the balanced
-// kernel.  With `work` the time of the padded product at
-// three quarters of the peak, the configuration loses the idle part of its
-// last round of workgroups and, when it splits K, a reduction launch and its
-// traffic; the balanced kernel loses a few us, and a share of its time, to cut
-// tiles.  Measured, configuration against balanced: FP64 2874x1426x1995 336 /
-// 290 us, 2048x700x3000 187 / 159, 1573x721x1984 109 / 104, 1000x777x1203 56 /
-// 50; FP32 1645x1384x2732 132 / 123, 779x796x1129 33 / 25; on the other side
-// FP64 2887x1224x505 75 / 83, 2629x660x760 60 / 63, FP32 2801x2411x710 96 / 106.
-static bool balanced_pays(bool f64, int64_t m, int64_t n, int64_t k, int config) {
-  if (many_large_tiles(f64, m, n)) return false;
+// Times (us) of a plain product on configuration `config` and on the balanced
+// kernel, by what each does: a fixed part, the chain of k slices of one
+// workgroup, those of the workgroups that share a CU, the tiles, and the sums
+// of parts (a reduction launch and its traffic; one after another by the last
+// workgroup of a tile).  Coefficients by least squares of the relative error
+// over 1070 products, FP32 and FP64, all four op pairs, 384 to 3000 on a side
+// and skinny ones with k to 60,000: off by 5 to 7% (rms).
+static double config_time(bool f64, int64_t m, int64_t n, int64_t k, int config) {
   int tile, splits;
   config_decode(config, &tile, &splits);
-  auto count = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
-  const int64_t wgs = count(kTileM[tile], kTileN[tile]) * splits;
-  const double idle = (double)((wgs + kCUs - 1) / kCUs * kCUs) / (double)wgs - 1.0;
-  const double flops_per_us = f64 ? 59e6 : 118e6;
-  const double work = 2.0 * (double)(count(64, 64) * 4096) * (double)k / flops_per_us;
-  const double reduce = splits > 1 ? 2.0 + (double)splits * (double)m * (double)n * (f64 ? 8 : 4) / 4e6 : 0.0;
-  return idle * work + reduce >= (f64 ? 10.0 + 0.06 * work : 4.0 + 0.10 * work);
+  const int64_t bk = f64 ? 16 : 32;
+  const int64_t slices = ((k + splits - 1) / splits + bk - 1) / bk;
+  const int64_t parts = (k + slices * bk - 1) / (slices * bk);
+  const int64_t bm = kTileM[tile], bn = kTileN[tile];
+  const double rounds = (double)((((m + bm - 1) / bm) * ((n + bn - 1) / bn) * parts + kCUs - 1) / kCUs);
+  const double area = (double)(bm * bn) / 4096.0, chain = (double)slices;
+  const double sums = parts > 1 ? (double)parts * (double)m * (double)n * (f64 ? 8e-6 : 4e-6) : 0.0;
+  return f64 ? 6.46 + chain * (0.159 * std::sqrt(area) + 0.485 * area * rounds) + 0.108 * rounds +
+                   (parts > 1 ? 1.54 + 0.241 * sums : 0.0)
+             : 6.96 + chain * (0.165 * std::sqrt(area) + 0.471 * area * rounds) + 0.428 * rounds +
+                   (parts > 1 ? 1.09 + 0.502 * sums : 0.0);
+}
+static double balanced_time(bool f64, int64_t m, int64_t n, int64_t k) {
+  const int64_t b = kBalancedTile, bk = f64 ? 16 : 32;
+  const int64_t tiles = ((m + b - 1) / b) * ((n + b - 1) / b), units = tiles * ((k + bk - 1) / bk);
+  const double groups = balanced_groups(units), run = (double)units / groups;
+  const double parts = std::max(groups / (double)tiles, 1.0) - 1.0, shared = std::max(groups / kCUs - 1.0, 0.0);
+  return f64 ? 9.78 + run * (0.590 + 0.592 * shared) + 0.456 * parts + 3.07 * (double)tiles / kCUs
+             : 8.15 + run * (0.592 + 0.691 * shared) + 0.331 * parts + 3.53 * (double)tiles / kCUs;
+}
+
+// Whether a plain product leaves configuration `config` for the balanced
+// kernel: where that is expected to take 7% (FP32, whose estimates are wider:
+// 10%) and 3.5 us less.  Of 367 other products that pass, 5 were slower than on
+// their configuration, by 2 to 7%; the rest took 0.83 times as long in the mean
+// (FP64 130 x 130 x 20,000 115 -> 62 us, 1000x777x1203 54 -> 50, FP32
+// 779x796x1129 32 -> 25).  On the other side: FP64 2683x1057x2702 281 against
+// 329 us, 64 x 64 x 2048 18 / 25, FP32 903x1358x409 20 / 24.
+static bool balanced_pays(bool f64, int64_t m, int64_t n, int64_t k, int config) {
+  if (many_large_tiles(f64, m, n)) return false;
+  const double t = config_time(f64, m, n, k, config);
+  return balanced_time(f64, m, n, k) < std::min((f64 ? 0.93 : 0.90) * t, t - 3.5);
 }
 
 template <typename T>
