@@ -707,26 +707,28 @@ template bool tri_product<double>(bool, bool, bool, bool, int64_t, int64_t, doub
                                   const double*, int64_t, double*, int64_t, hipStream_t, eh_status*);
 
 template <typename T>
-bool complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,
-                       const T* B3, int64_t ldb3, T beta, T* C, int64_t ldc, int prec, hipStream_t stream,
-                       eh_status* st) {
+bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb3, int prec) {
   if (std::is_same<T, float>::value && prec == EH_PREC_AUTO) prec = default_sgemm_precision();
   if (prec != EH_PREC_PLAIN && prec != EH_PREC_AUTO) return false;
-  if (n == 1 || many_large_tiles(std::is_same<T, double>::value, 2 * m, n) || !operand_fits<T>(ta, ta ? m : 2 * m, ta ? 2 * k : k, 2 * lda) ||
-      !operand_fits<T>(true, n, 2 * k, ldb3))
-    return false;
+  return n > 1 && !many_large_tiles(std::is_same<T, double>::value, 2 * m, n) &&
+         operand_fits<T>(ta, ta ? m : 2 * m, ta ? 2 * k : k, 2 * lda) && operand_fits<T>(true, n, 2 * k, ldb3);
+}
+template bool complex_a_in_place<float>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int);
+template bool complex_a_in_place<double>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int);
+
+template <typename T>
+eh_status complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,
+                            const T* B3, int64_t ldb3, T beta, T* C, int64_t ldc, hipStream_t stream) {
   GemmParams<T> p = product_params<T>(false, false, 2 * m, n, 2 * k, ar, A, lda, B3, ldb3, beta, C, 2 * ldc);
   p.bytesA = (uint32_t)((ta ? (uint64_t)(m - 1) * lda + k : (uint64_t)(k - 1) * lda + m) * 2 * sizeof(T));
   p.alpha_im = ai;
   p.conj = conj;
-  *st = launch_balanced<T>(p, kComplexA, ta, false, stream);
-  return true;
+  return launch_balanced<T>(p, kComplexA, ta, false, stream);
 }
-template bool complex_a_product<float>(bool, bool, int64_t, int64_t, int64_t, float, float, const float*, int64_t,
-                                       const float*, int64_t, float, float*, int64_t, int, hipStream_t, eh_status*);
-template bool complex_a_product<double>(bool, bool, int64_t, int64_t, int64_t, double, double, const double*, int64_t,
-                                        const double*, int64_t, double, double*, int64_t, int, hipStream_t,
-                                        eh_status*);
+template eh_status complex_a_product<float>(bool, bool, int64_t, int64_t, int64_t, float, float, const float*, int64_t,
+                                            const float*, int64_t, float, float*, int64_t, hipStream_t);
+template eh_status complex_a_product<double>(bool, bool, int64_t, int64_t, int64_t, double, double, const double*,
+                                             int64_t, const double*, int64_t, double, double*, int64_t, hipStream_t);
 
 // Tickets for a split matrix-vector product, or nullptr (the sums are the same
 // bits either way): in a captured call and in the fixed scratch, and for more

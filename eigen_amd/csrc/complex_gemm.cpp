@@ -38,27 +38,27 @@ eh_status run(int dtype, int opa, int opb, int64_t m, int64_t n, int64_t k, cons
     if (vanishes) return EH_SUCCESS;
     beff = T(1);
   }
-  const T* B3 = B;
-  int64_t ldb3 = 2 * ldb;
-  StreamTemp tb;
-  if (opb != EH_OP_N) {
-    eh_status st = tb.get((size_t)2 * k * n * sizeof(T), s, "complex product temporary");
+  // one temporary for whatever is repacked: two took 19 us more per call
+  const bool ta = opa != EH_OP_N, pack_b = opb != EH_OP_N;
+  const int64_t ldb3 = pack_b ? 2 * k : 2 * ldb;
+  const bool in_place = complex_a_in_place<T>(ta, m, n, k, lda, ldb3, prec);
+  const size_t a3 = in_place ? 0 : (size_t)4 * m * k, b3 = pack_b ? (size_t)2 * k * n : 0;
+  StreamTemp t;
+  if (a3 + b3 > 0) {
+    eh_status st = t.get((a3 + b3) * sizeof(T), s, "complex product temporary");
     if (st != EH_SUCCESS) return st;
-    T* P = static_cast<T*>(tb.ptr);
-    hipError_t e = launch_complex_pack_b<T>(B, ldb, (int)k, (int)n, true, opb == EH_OP_C, P, 2 * k, s);
+  }
+  T* A3 = static_cast<T*>(t.ptr);
+  const T* B3 = B;
+  if (pack_b) {
+    T* P = A3 + a3;
+    hipError_t e = launch_complex_pack_b<T>(B, ldb, (int)k, (int)n, true, opb == EH_OP_C, P, ldb3, s);
     if (e != hipSuccess) return hip_fail(e, "complex pack launch");
     B3 = P;
-    ldb3 = 2 * k;
   }
-  eh_status st = EH_SUCCESS;
-  if (complex_a_product<T>(opa != EH_OP_N, opa == EH_OP_C, m, n, k, ar, ai, A, lda, B3, ldb3, beff, C, ldc, prec, s,
-                           &st))
-    return st;
-  StreamTemp ta;
-  st = ta.get((size_t)4 * m * k * sizeof(T), s, "complex product temporary");
-  if (st != EH_SUCCESS) return st;
-  T* A3 = static_cast<T*>(ta.ptr);
-  hipError_t e = launch_complex_pack_a<T>(A, lda, (int)m, (int)k, opa != EH_OP_N, opa == EH_OP_C, ar, ai, A3, 2 * m, s);
+  if (in_place)
+    return complex_a_product<T>(ta, opa == EH_OP_C, m, n, k, ar, ai, A, lda, B3, ldb3, beff, C, ldc, s);
+  hipError_t e = launch_complex_pack_a<T>(A, lda, (int)m, (int)k, ta, opa == EH_OP_C, ar, ai, A3, 2 * m, s);
   if (e != hipSuccess) return hip_fail(e, "complex pack launch");
   const T one = T(1);
   return gemm_dispatch(dtype, EH_OP_N, EH_OP_N, 2 * m, n, 2 * k, &one, A3, 2 * m, B3, ldb3, &beff, C, 2 * ldc, prec, -1,

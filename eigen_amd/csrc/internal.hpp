@@ -141,13 +141,14 @@ template <typename T>
 bool tri_product(bool left, bool tri_t, bool lower, bool unit, int64_t order, int64_t other, T alpha, const T* E,
                  int64_t lde, const T* X, int64_t ldx, T* C, int64_t ldc, hipStream_t stream, eh_status* st);
 // Complex product with A read in place (interleaved pairs, lda and ldc in
-// pairs) and B3 the real 2k x n form of op(B); beta real.  Returns false
-// (nothing done) for split precisions, one column, products large enough for
-// 128x128 tiles, and operands past 32-bit addressing.
+// pairs) and B3 the real 2k x n form of op(B); beta real.  Only where
+// complex_a_in_place says so: not for split precisions, one column, products
+// large enough for 128x128 tiles, and operands past 32-bit addressing.
 template <typename T>
-bool complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,
-                       const T* B3, int64_t ldb3, T beta, T* C, int64_t ldc, int prec, hipStream_t stream,
-                       eh_status* st);
+bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb3, int prec);
+template <typename T>
+eh_status complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,
+                            const T* B3, int64_t ldb3, T beta, T* C, int64_t ldc, hipStream_t stream);
 eh_status gemm_dispatch(int dtype, int opa, int opb, int64_t m, int64_t n, int64_t k, const void* alpha,
                         const void* A, int64_t lda, const void* B, int64_t ldb, const void* beta, void* C,
                         int64_t ldc, int prec, int config, void* stream);
