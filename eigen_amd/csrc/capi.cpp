@@ -686,6 +686,11 @@ static bool balanced_pays(bool f64, int64_t m, int64_t n, int64_t k, int config)
   return balanced_time(f64, m, n, k) < std::min((f64 ? 0.93 : 0.90) * t, t - 3.5);
 }
 
+// Whether products leave the planner's configurations for the small and
+// balanced kernels: a caller who chose another planner, or a network of its own,
+// gets what that chooses.
+static bool own_rules() { return tune_mode() == EH_TUNE_MLP && !mlp_installed(); }
+
 template <typename T>
 bool tri_product(bool left, bool tri_t, bool lower, bool unit, int64_t order, int64_t other, T alpha, const T* E,
                  int64_t lde, const T* X, int64_t ldx, T* C, int64_t ldc, hipStream_t stream, eh_status* st) {
@@ -710,6 +715,7 @@ template <typename T>
 bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb3, int prec) {
   if (std::is_same<T, float>::value && prec == EH_PREC_AUTO) prec = default_sgemm_precision();
   if (prec != EH_PREC_PLAIN && prec != EH_PREC_AUTO) return false;
+  if (!own_rules()) return false;
   return n > 1 && !many_large_tiles(std::is_same<T, double>::value, 2 * m, n) &&
          operand_fits<T>(ta, ta ? m : 2 * m, ta ? 2 * k : k, 2 * lda) && operand_fits<T>(true, n, 2 * k, ldb3);
 }
@@ -797,11 +803,6 @@ static bool small_product(int64_t m, int64_t n, int64_t k) {
   const int64_t tiles = ((m + kSmallTile - 1) / kSmallTile) * ((n + kSmallTile - 1) / kSmallTile);
   return tiles <= 2 * kCUs && (k <= 512 || (k <= 1024 && tiles >= kCUs / 4));
 }
-
-// Whether products leave the planner's configurations for the small and
-// balanced kernels: a caller who chose another planner, or a network of its own,
-// gets what that chooses.
-static bool own_rules() { return tune_mode() == EH_TUNE_MLP && !mlp_installed(); }
 
 // Kernel of a plain-precision product, and its configuration unless small.
 template <typename T>

@@ -1,0 +1,54 @@
+"""Complex products that leave A in place do so only under the default planner
+and outside a capture: elsewhere they repack A and are, bit for bit, the real
+product of the 2x2 block form that eh_gemm runs in the same way.  Operands are
+not integers, and the in-place form's other order of summation shows in the
+last bits (checked, so that the comparison means something)."""
+import pytest
+import torch
+
+import eigen_amd as E
+
+pytestmark = pytest.mark.gpu
+
+M, N, K = 256, 200, 700
+
+
+def operands(seed):
+    g = torch.Generator("cuda").manual_seed(seed)
+    a = torch.view_as_complex(torch.rand(K, M, 2, generator=g, dtype=torch.float64, device="cuda") - 0.5)  # column-major M x K
+    b = torch.view_as_complex(torch.rand(N, K, 2, generator=g, dtype=torch.float64, device="cuda") - 0.5)
+    a3 = torch.empty(2 * K, 2 * M, dtype=torch.float64, device="cuda")  # column-major 2M x 2K
+    a3[0::2, 0::2], a3[0::2, 1::2] = a.real, a.imag
+    a3[1::2, 0::2], a3[1::2, 1::2] = -a.imag, a.real
+    return a.contiguous(), b.contiguous(), a3
+
+
+def complex_product(a, b, c, stream=None):
+    E.gemm_complex(E.F64, 0, 0, M, N, K, 1.0, a, M, b, K, 0.0, c, M, prec=E.PREC_PLAIN, stream=stream)
+
+
+def real_product(a3, b, c, stream=None):
+    E.gemm(E.F64, 0, 0, 2 * M, N, 2 * K, 1.0, a3, 2 * M, torch.view_as_real(b), 2 * K, 0.0, c, 2 * M,
+           prec=E.PREC_PLAIN, stream=stream)
+
+
+def both(a, b, a3):
+    c, r = torch.zeros(N, M, dtype=torch.complex128, device="cuda"), torch.zeros(N, 2 * M, dtype=torch.float64, device="cuda")
+    complex_product(a, b, c)
+    real_product(a3, b, r)
+    torch.cuda.synchronize()
+    return torch.view_as_real(c).reshape(N, 2 * M), r
+
+
+def test_other_planner(gpu):
+    ops = operands(1)
+    prev = E.lib().eh_get_tune_mode()
+    try:
+        E.set_tune_mode(E.TUNE_HEURISTIC)
+        c, want = both(*ops)
+        assert torch.equal(c, want)
+        E.set_tune_mode(E.TUNE_MLP)
+        c, _ = both(*ops)
+        assert not torch.equal(c, want) and torch.allclose(c, want, rtol=0, atol=1e-12)
+    finally:
+        E.set_tune_mode(prev)
