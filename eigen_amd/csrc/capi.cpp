@@ -585,8 +585,8 @@ static eh_status launch_product(bool ta, bool tb, int64_t m, int64_t n, int64_t 
 // Launches p on the balanced kernel: with tickets and slots from the stream's
 // workspace or the installed fixed scratch, or (one workgroup per tile)
 // without, in a captured call: it may be replayed beside other work of this
-// stream's workspace.  (A plain product then keeps its configuration, run_gemm
-// below.)
+// stream's workspace.  (Plain and complex products then keep the planner's
+// configuration; a triangular product runs uncut.)
 static bool balanced_workspace_allowed(hipStream_t stream) {
   return fixed_scratch_active() || !stream_capturing(stream);
 }
@@ -712,15 +712,18 @@ template bool tri_product<double>(bool, bool, bool, bool, int64_t, int64_t, doub
                                   const double*, int64_t, double*, int64_t, hipStream_t, eh_status*);
 
 template <typename T>
-bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb3, int prec) {
+bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb3, int prec,
+                        hipStream_t stream) {
   if (std::is_same<T, float>::value && prec == EH_PREC_AUTO) prec = default_sgemm_precision();
   if (prec != EH_PREC_PLAIN && prec != EH_PREC_AUTO) return false;
-  if (!own_rules()) return false;
+  // in a captured call, one workgroup per tile is several times slower than the
+  // planner's split K (complex128 64 x 64 x 2048: 178 against 42 us)
+  if (!own_rules() || !balanced_workspace_allowed(stream)) return false;
   return n > 1 && !many_large_tiles(std::is_same<T, double>::value, 2 * m, n) &&
          operand_fits<T>(ta, ta ? m : 2 * m, ta ? 2 * k : k, 2 * lda) && operand_fits<T>(true, n, 2 * k, ldb3);
 }
-template bool complex_a_in_place<float>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int);
-template bool complex_a_in_place<double>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int);
+template bool complex_a_in_place<float>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int, hipStream_t);
+template bool complex_a_in_place<double>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int, hipStream_t);
 
 template <typename T>
 eh_status complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,

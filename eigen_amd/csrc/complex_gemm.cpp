@@ -41,7 +41,7 @@ eh_status run(int dtype, int opa, int opb, int64_t m, int64_t n, int64_t k, cons
   // one temporary for whatever is repacked: two took 19 us more per call
   const bool ta = opa != EH_OP_N, pack_b = opb != EH_OP_N;
   const int64_t ldb3 = pack_b ? 2 * k : 2 * ldb;
-  const bool in_place = complex_a_in_place<T>(ta, m, n, k, lda, ldb3, prec);
+  const bool in_place = complex_a_in_place<T>(ta, m, n, k, lda, ldb3, prec, s);
   const size_t a3 = in_place ? 0 : (size_t)4 * m * k, b3 = pack_b ? (size_t)2 * k * n : 0;
   StreamTemp t;
   if (a3 + b3 > 0) {

@@ -52,3 +52,26 @@ def test_other_planner(gpu):
         assert not torch.equal(c, want) and torch.allclose(c, want, rtol=0, atol=1e-12)
     finally:
         E.set_tune_mode(prev)
+
+
+def test_captured(gpu):
+    a, b, a3 = operands(2)
+    c, r = torch.zeros(N, M, dtype=torch.complex128, device="cuda"), torch.zeros(N, 2 * M, dtype=torch.float64, device="cuda")
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        complex_product(a, b, c, s.cuda_stream)
+        real_product(a3, b, r, s.cuda_stream)
+        torch.cuda.synchronize()
+        g.capture_begin()
+        complex_product(a, b, c, s.cuda_stream)
+        real_product(a3, b, r, s.cuda_stream)
+        g.capture_end()
+    for _ in range(3):
+        c.zero_()
+        r.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(torch.view_as_real(c).reshape(N, 2 * M), r)
+        eager, _ = both(a, b, a3)
+        assert torch.allclose(eager, r, rtol=0, atol=1e-12)
