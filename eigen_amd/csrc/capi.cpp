@@ -719,8 +719,24 @@ bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, i
   // in a captured call, one workgroup per tile is several times slower than the
   // planner's split K (complex128 64 x 64 x 2048: 178 against 42 us)
   if (!own_rules() || !balanced_workspace_allowed(stream)) return false;
-  return n > 1 && !many_large_tiles(std::is_same<T, double>::value, 2 * m, n) &&
-         operand_fits<T>(ta, ta ? m : 2 * m, ta ? 2 * k : k, 2 * lda) && operand_fits<T>(true, n, 2 * k, ldb3);
+  constexpr bool f64 = std::is_same<T, double>::value;
+  if (n == 1 || many_large_tiles(f64, 2 * m, n) || !operand_fits<T>(ta, ta ? m : 2 * m, ta ? 2 * k : k, 2 * lda) ||
+      !operand_fits<T>(true, n, 2 * k, ldb3))
+    return false;
+  // With tiles enough, in place (complex64 1875x909x1638 228 us, repacked 298).
+  // A tile in more than four parts is the other side: the last workgroup adds
+  // them one after another (complex64 4 x 4096 x 4096 149 us repacked, 166 in
+  // place, complex128 2 x 6 x 4620 63 and 71).  There repacking costs a pass over
+  // A, and the host the pass's launch and a temporary: small products take 37 us.
+  const int64_t b = kBalancedTile, bk = f64 ? 16 : 32;
+  const int64_t tiles = ((2 * m + b - 1) / b) * ((n + b - 1) / b);
+  if (balanced_groups(tiles * ((2 * k + bk - 1) / bk)) <= 4 * tiles) return true;
+  const double t = balanced_time(f64, 2 * m, n, 2 * k);
+  if (t < 37.0) return true;
+  int config = 0;
+  if (plan_config(f64 ? EH_F64 : EH_F32, EH_OP_N, EH_OP_N, 2 * m, n, 2 * k, &config) != EH_SUCCESS) return false;
+  const double pass = 3.0 + 6.0 * (double)m * (double)k * sizeof(T) / 4e6;
+  return t < std::max(config_time(f64, 2 * m, n, 2 * k, config) + pass, 37.0);
 }
 template bool complex_a_in_place<float>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int, hipStream_t);
 template bool complex_a_in_place<double>(bool, int64_t, int64_t, int64_t, int64_t, int64_t, int, hipStream_t);

@@ -144,9 +144,11 @@ bool tri_product(bool left, bool tri_t, bool lower, bool unit, int64_t order, in
 // pairs) and B3 the real 2k x n form of op(B); beta real.  Only where
 // complex_a_in_place says so: not for split precisions, one column, products
 // large enough for 128x128 tiles, operands past 32-bit addressing, captured
-// calls, and under another planner than the compiled-in network.
+// calls, under another planner than the compiled-in network, and where a copy
+// of A and the planner's kernel are faster.
 template <typename T>
-bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb3, int prec, hipStream_t stream);
+bool complex_a_in_place(bool ta, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb3, int prec,
+                        hipStream_t stream);
 template <typename T>
 eh_status complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k, T ar, T ai, const T* A, int64_t lda,
                             const T* B3, int64_t ldb3, T beta, T* C, int64_t ldc, hipStream_t stream);

@@ -1,5 +1,5 @@
-"""Complex products that leave A in place do so only under the default planner
-and outside a capture: elsewhere they repack A and are, bit for bit, the real
+"""Complex products that leave A in place do so only under the default planner,
+outside a capture and where they have tiles enough: elsewhere they repack A and are, bit for bit, the real
 product of the 2x2 block form that eh_gemm runs in the same way.  Operands are
 not integers, and the in-place form's other order of summation shows in the
 last bits (checked, so that the comparison means something)."""
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 M, N, K = 256, 200, 700
 
 
-def operands(seed):
+def operands(seed, M=M, N=N, K=K):
     g = torch.Generator("cuda").manual_seed(seed)
     a = torch.view_as_complex(torch.rand(K, M, 2, generator=g, dtype=torch.float64, device="cuda") - 0.5)  # column-major M x K
     b = torch.view_as_complex(torch.rand(N, K, 2, generator=g, dtype=torch.float64, device="cuda") - 0.5)
@@ -24,15 +24,18 @@ def operands(seed):
 
 
 def complex_product(a, b, c, stream=None):
+    (K, M), N = a.shape, len(b)
     E.gemm_complex(E.F64, 0, 0, M, N, K, 1.0, a, M, b, K, 0.0, c, M, prec=E.PREC_PLAIN, stream=stream)
 
 
 def real_product(a3, b, c, stream=None):
+    (K, M), N = (x // 2 for x in a3.shape), len(b)
     E.gemm(E.F64, 0, 0, 2 * M, N, 2 * K, 1.0, a3, 2 * M, torch.view_as_real(b), 2 * K, 0.0, c, 2 * M,
            prec=E.PREC_PLAIN, stream=stream)
 
 
 def both(a, b, a3):
+    (K, M), N = a.shape, len(b)
     c, r = torch.zeros(N, M, dtype=torch.complex128, device="cuda"), torch.zeros(N, 2 * M, dtype=torch.float64, device="cuda")
     complex_product(a, b, c)
     real_product(a3, b, r)
@@ -75,3 +78,9 @@ def test_captured(gpu):
         assert torch.equal(torch.view_as_real(c).reshape(N, 2 * M), r)
         eager, _ = both(a, b, a3)
         assert torch.allclose(eager, r, rtol=0, atol=1e-12)
+
+
+def test_few_tiles(gpu):
+    """Two tiles of deep k: in place, one workgroup would add 64 parts each."""
+    c, want = both(*operands(3, 64, 64, 2048))
+    assert torch.equal(c, want)
