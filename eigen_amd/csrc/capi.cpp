@@ -586,10 +586,9 @@ static eh_status launch_product(bool ta, bool tb, int64_t m, int64_t n, int64_t 
 // workspace or the installed fixed scratch, or (one workgroup per tile)
 // without, in a captured call: it may be replayed beside other work of this
 // stream's workspace.  (Plain and complex products then keep the planner's
-// configuration; a triangular product runs uncut.)
-static bool balanced_workspace_allowed(hipStream_t stream) {
-  return fixed_scratch_active() || !stream_capturing(stream);
-}
+// configuration, also with the fixed scratch, so that eh_gemm_noalloc gives
+// eh_gemm's bits either way; a triangular product runs uncut.)
+static bool balanced_workspace_allowed(hipStream_t stream) { return !stream_capturing(stream); }
 
 // Workgroups the balanced kernel runs: it fits three to a CU, and short runs
 // do better as two longer ones (FP64 1000x777x1203, 62 slices per CU: 50.1
@@ -617,7 +616,7 @@ eh_status launch_balanced(GemmParams<T> p, int mode, bool ta, bool tb, hipStream
     const size_t slots = (size_t)groups * 2 * b * b * sizeof(T);
     if (fixed_scratch_active()) {
       // nothing in the fixed scratch outlives a call: the tickets lie behind
-      // the slots and are cleared first (a kernel, so a capture may hold it)
+      // the slots and are cleared first
       eh_status st = workspace_get(stream, slots + (size_t)tiles * sizeof(unsigned), &lease, &ws);
       if (st != EH_SUCCESS) return st;
       tickets = reinterpret_cast<unsigned*>(static_cast<unsigned char*>(ws) + slots);

@@ -104,7 +104,9 @@ typedef enum eh_tune_mode {
 /* C = alpha*op(A)*op(B) + beta*C.  m x n result, inner dimension k.
  * beta == 0: C is written without being read (NaN/Inf in C are discarded).
  * alpha == 0 or k == 0: A and B are not read; C = beta*C.
- * m == 0 or n == 0: nothing happens. */
+ * m == 0 or n == 0: nothing happens.
+ * A call that is captured into a graph may run another kernel than one that is
+ * not (eh_plan_kernel) and round differently. */
 eh_status eh_gemm(eh_dtype dtype, eh_op opa, eh_op opb, int64_t m, int64_t n, int64_t k, const void* alpha,
                   const void* A, int64_t lda, const void* B, int64_t ldb, const void* beta, void* C, int64_t ldc,
                   eh_precision prec, void* stream);
@@ -112,7 +114,8 @@ eh_status eh_gemm(eh_dtype dtype, eh_op opa, eh_op opb, int64_t m, int64_t n, in
 /* eh_gemm with no device allocation.  No counterpart in the reference: for
  * callers that cannot allocate device memory (code under hipGraph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments,
- * dispatch, kernels and results (bit for bit) as eh_gemm; the workspace
+ * dispatch, kernels and results (bit for bit) as eh_gemm called the same way,
+ * both captured into a graph or neither; the workspace
  * eh_gemm would take from its per-stream pool (split-K partial sums, the
  * packed bf16 planes of a split-precision product, matrix-vector partial
  * sums) is instead one fixed device array of EH_NOALLOC_SCRATCH_BYTES per
