@@ -812,7 +812,11 @@ static void launch_small_t(bool ta, bool tb, const void* A, int64_t lda, int64_t
   auto f = k < EPC        ? (one ? launch_small_vec<T, KS, 0, 1> : launch_small_vec<T, KS, 0, 2>)
            : k % EPC == 0 ? (one ? launch_small_vec<T, KS, 1, 1> : launch_small_vec<T, KS, 1, 2>)
                           : (one ? launch_small_vec<T, KS, 2, 1> : launch_small_vec<T, KS, 2, 2>);
-  f(ta, tb, A, lda, sa, B, ldb, sb, C, ldc, sc, m, n, k, alpha, beta, count, s);
+  // a launch holds fewer than 2^32 threads: 2^25 products at a time
+  constexpr int64_t kMost = 1 << 25;
+  for (int64_t p = 0; p < count; p += kMost)
+    f(ta, tb, static_cast<const T*>(A) + p * sa, lda, sa, static_cast<const T*>(B) + p * sb, ldb, sb,
+      static_cast<T*>(C) + p * sc, ldc, sc, m, n, k, alpha, beta, std::min(kMost, count - p), s);
 }
 
 }  // namespace eh

@@ -47,3 +47,16 @@ def test_one_wave_exact(gpu, dtype, code, ta, tb, m, n, k):
         inner[:, :, :m] = 0
         start[:, :n * ldc].reshape(count, n, ldc)[:, :, :m] = 0
         assert np.array_equal(got, start, equal_nan=True)  # nothing else is written
+
+
+@pytest.mark.parametrize("m", [17, 5])
+def test_one_wave_past_one_grid(gpu, m):
+    """More products than one launch of a wave each can hold (2^32 threads)."""
+    count = (1 << 26) + 5
+    a = torch.arange(count * m, device="cuda", dtype=torch.int32).remainder_(251).float()
+    b = torch.arange(count, device="cuda", dtype=torch.int32).remainder_(13).float()
+    c = torch.full((count * m,), float("nan"), device="cuda")
+    E.gemm_batched_strided(E.F32, 0, 0, m, 1, 1, 2.0, a, m, m, b, 1, 1, 0.0, c, m, m, count)
+    torch.cuda.synchronize()
+    a.view(count, m).mul_(2.0 * b[:, None])
+    assert torch.equal(a, c)
