@@ -765,10 +765,14 @@ static unsigned* gemv_tickets(const GemvPlan& g, hipStream_t stream, WorkspaceLe
   return tickets;
 }
 
+// Rows of A^T x in one launch, 32 to a workgroup of 256 threads: a grid holds
+// fewer than 2^32 threads.
+constexpr int64_t kGemvMaxRows = 1 << 28;
+
 // A product with one output column (n == 1) or row (m == 1) is a
 // matrix-vector product: C^T = op(B)^T op(A)^T turns the row case into the
 // column case.  Returns false (nothing launched) when the matrix spans 4 GB
-// or more; the tiled path then handles it.
+// or more, or has more rows than a launch takes; the tiled path then handles it.
 template <typename T>
 static bool vector_product(int opa, int opb, int64_t m, int64_t n, int64_t k, T alpha, const T* A, int64_t lda,
                            const T* B, int64_t ldb, T beta, T* C, int64_t ldc, hipStream_t stream, eh_status* st) {
@@ -795,7 +799,7 @@ static bool vector_product(int opa, int opb, int64_t m, int64_t n, int64_t k, T 
   }
   const uint64_t extent =
       ((trans ? (uint64_t)(rows - 1) * ldm + k : (uint64_t)(k - 1) * ldm + rows) + 64) * sizeof(T);
-  if (extent >= kMaxExtent) return false;
+  if (extent >= kMaxExtent || (trans && rows > kGemvMaxRows)) return false;
   const GemvPlan g = gemv_plan(trans, rows, (int)k, (int)sizeof(T));
   void* ws = nullptr;
   WorkspaceLease lease;
@@ -929,7 +933,7 @@ static eh_status gemv_run(bool trans, int64_t rows, int64_t k, T alpha, const T*
     return e == hipSuccess ? EH_SUCCESS : hip_fail(e, "scale launch");
   }
   const uint64_t extent = ((trans ? (uint64_t)(rows - 1) * lda + k : (uint64_t)(k - 1) * lda + rows) + 64) * sizeof(T);
-  if (extent >= kMaxExtent) {
+  if (extent >= kMaxExtent || (trans && rows > kGemvMaxRows)) {
     if (!trans && k > 1) {
       const int64_t h = k / 2;
       eh_status st = gemv_run<T>(false, rows, h, alpha, A, lda, x, incx, beta, y, incy, s);
@@ -1181,7 +1185,9 @@ eh_status eh_plan_kernel(eh_dtype dtype, eh_op opa, eh_op opb, int64_t m, int64_
   if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return fail(EH_ERR_UNSUPPORTED, "m, n, k must fit int32");
   const int64_t lda = opa == EH_OP_N ? m : k, ldb = opb == EH_OP_N ? k : n;
   const uint64_t es = dtype == EH_F64 ? sizeof(double) : sizeof(float);
-  if ((m == 1 || n == 1) && ((uint64_t)std::max(m, n) * (uint64_t)k + 64) * es < kMaxExtent) {
+  const bool trans = n == 1 ? opa != EH_OP_N : opb == EH_OP_N;
+  if ((m == 1 || n == 1) && ((uint64_t)std::max(m, n) * (uint64_t)k + 64) * es < kMaxExtent &&
+      !(trans && std::max(m, n) > kGemvMaxRows)) {
     *kernel = EH_KERNEL_VECTOR;
     return EH_SUCCESS;
   }

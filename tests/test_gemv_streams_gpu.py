@@ -110,3 +110,18 @@ def test_gemv_t_short_rows_exact(gpu, dtype, code, m, n, pad, incx, incy):
     torch.cuda.synchronize()
     got = dy.cpu().numpy()[::abs(incy)]
     assert np.array_equal((got if incy > 0 else got[::-1]).astype(np.float64), want)
+
+
+def test_gemv_t_past_one_grid(gpu):
+    """More rows of A^T x than one launch of 32 to a workgroup holds (2^32 threads)."""
+    n = 600_000_001
+    a = torch.arange(n, device="cuda", dtype=torch.int32).remainder_(251).float()
+    x = torch.full((1,), 3.0, device="cuda")
+    y = torch.full((n,), float("nan"), device="cuda")
+    E.gemv(E.F32, 1, 1, n, 2.0, a, 1, x, 1, 0.0, y, 1)
+    torch.cuda.synchronize()
+    assert torch.equal(a.mul_(6.0), y)
+    y.fill_(float("nan"))
+    E.gemm(E.F32, 0, 0, 1, n, 1, 0.5, x, 1, a, 1, 0.0, y, 1, prec=E.PREC_PLAIN)
+    torch.cuda.synchronize()
+    assert torch.equal(a.mul_(1.5), y)
