@@ -106,6 +106,7 @@ struct TrtriParams {
   int mt, lower, unit, order;
   T* W;
   int conj = 0;
+  int columns = 0;  // real types: the inverses column-major also when mt
 };
 template <typename T>
 hipError_t launch_trtri(const TrtriParams<T>& p, hipStream_t s);
@@ -125,6 +126,12 @@ struct TrsmPanelParams {
   int ta, lower, sz, ncols;
   T alpha;
 };
+// The panels of a triangle of order `order` whose rows are contiguous (E(i, k) =
+// A[k + i*lda]), turned: E(i, k) of the panel at d (a multiple of kTrsmPanel) at
+// D[d*ldd + (i - d) + (k - d)*ldd], its 64 x 64 diagonal blocks left out.  ldd =
+// kTrsmPanel, or with a single panel its order rounded up to 64.
+template <typename T>
+hipError_t launch_turn_panels(const T* A, int64_t lda, int order, bool lower, T* D, int ldd, hipStream_t s);
 template <typename T>
 hipError_t launch_trsm_panel(const TrsmPanelParams<T>& p, hipStream_t s);
 // D (m x n, leading dimension m) = B.

@@ -118,12 +118,21 @@ struct TrsmWork {
   int64_t leaf;  // order of the inverted blocks
 };
 
+// What a real solve prepares: the inverses of the diagonal blocks of E (left) or
+// E^T (right), and where that operator's rows are contiguous in FP64, its panels
+// turned (launch_turn_panels; else null).
+template <typename T>
+struct TrsmReal {
+  const T* inv;
+  const T* turned;
+  int64_t ldt;
+};
+
 // E X = alpha*B (left) or X E = alpha*B (right) in place for rows (columns) d0..
-// d0 + size of the system, real types; inv holds the inverses of the diagonal
-// blocks of E (left) or E^T (right).
+// d0 + size of the system, real types.
 template <typename T>
 eh_status trsm_panels(const Tri<T>& E, bool left, int64_t d0, int64_t size, int64_t other, T alpha, T* B, int64_t ldb,
-                      const T* inv, hipStream_t s) {
+                      const TrsmReal<T>& w, hipStream_t s) {
   const bool lower = left ? E.lower : !E.lower;  // triangle of the operator that acts on columns
   // rows r0.. of B = beta*B - (their part of E) * (solved rows d..)
   auto update = [&](int64_t r0, int64_t rows, int64_t d, int64_t sz, T beta) {
@@ -136,21 +145,21 @@ eh_status trsm_panels(const Tri<T>& E, bool left, int64_t d0, int64_t size, int6
     const int64_t h = half(size, kTrsmPanel);
     const int64_t d1 = lower ? d0 : d0 + h, n1 = lower ? h : size - h;  // solved first
     const int64_t d2 = lower ? d0 + h : d0, n2 = size - n1;
-    EH_TRY(trsm_panels(E, left, d1, n1, other, alpha, B, ldb, inv, s));
+    EH_TRY(trsm_panels(E, left, d1, n1, other, alpha, B, ldb, w, s));
     EH_TRY(update(d2, n2, d1, n1, alpha));
-    return trsm_panels(E, left, d2, n2, other, T(1), B, ldb, inv, s);
+    return trsm_panels(E, left, d2, n2, other, T(1), B, ldb, w, s);
   }
   const int64_t np = (size + kTrsmPanel - 1) / kTrsmPanel;
   for (int64_t q = 0; q < np; ++q) {
     const int64_t d = d0 + (lower ? q : np - 1 - q) * kTrsmPanel, sz = std::min<int64_t>(kTrsmPanel, d0 + size - d);
     TrsmPanelParams<T> p{};
-    p.A = E.diag(d);
-    p.inv = inv + d * kTrsmLeaf;
+    p.A = w.turned ? w.turned + d * w.ldt : E.diag(d);
+    p.inv = w.inv + d * kTrsmLeaf;
     p.B = left ? B + d : B + d * ldb;
-    p.lda = E.lda;
+    p.lda = w.turned ? w.ldt : E.lda;
     p.rs = left ? 1 : ldb;
     p.cs = left ? ldb : 1;
-    p.ta = left ? E.ta : !E.ta;
+    p.ta = w.turned ? 0 : left ? E.ta : !E.ta;
     p.lower = lower;
     p.sz = (int)sz;
     p.ncols = (int)other;
@@ -345,8 +354,13 @@ eh_status trsm_t(int side, int uplo, int transa, int diag, int64_t m, int64_t n,
   const int64_t blocks = (ka + leaf - 1) / leaf;
   const int64_t inv = blocks * leaf * leaf;
   const int64_t copy = !IsCplx<T>::value ? 0 : side == EH_LEFT ? leaf * n : m * leaf;
+  // real types solve X E = alpha*B as E^T X^T = alpha*B^T
+  const bool flip = !IsCplx<T>::value && side == EH_RIGHT;
+  const bool turn = std::is_same<T, double>::value && ta != flip && ka > 2 * leaf;
+  const int64_t ldt = std::min<int64_t>((ka + leaf - 1) / leaf * leaf, kTrsmPanel);
+  const int64_t turned = turn ? (ka + kTrsmPanel - 1) / kTrsmPanel * ldt * ldt : 0;
   StreamTemp t;
-  EH_TRY(t.get((size_t)(inv + copy) * sizeof(T), s, "level-3 temporary"));
+  EH_TRY(t.get((size_t)(inv + copy + turned) * sizeof(T), s, "level-3 temporary"));
   T* base = static_cast<T*>(t.ptr);
   StreamTemp dense;
   if constexpr (!IsCplx<T>::value) {
@@ -359,14 +373,18 @@ eh_status trsm_t(int side, int uplo, int transa, int diag, int64_t m, int64_t n,
       E.lda = lda = ka;
     }
   }
-  // real types solve X E = alpha*B as E^T X^T = alpha*B^T
-  const bool flip = !IsCplx<T>::value && side == EH_RIGHT;
   TrtriParams<T> tp{A, lda, (int)(E.ta != flip), (int)(E.lower != flip), (int)E.unit, (int)ka, base};
   tp.conj = E.conj;
+  tp.columns = turn;
   hipError_t e = launch_trtri<T>(tp, s);
   if (e != hipSuccess) return hip_fail(e, "diagonal block inversion launch");
   if constexpr (!IsCplx<T>::value) {
-    return trsm_panels<T>(E, side == EH_LEFT, 0, ka, side == EH_LEFT ? n : m, alpha, B, ldb, base, s);
+    if constexpr (std::is_same<T, double>::value) {
+      if (turn) e = launch_turn_panels<T>(A, lda, (int)ka, E.lower != flip, base + inv, (int)ldt, s);
+      if (e != hipSuccess) return hip_fail(e, "panel turning launch");
+    }
+    const TrsmReal<T> w{base, turn ? base + inv : nullptr, ldt};
+    return trsm_panels<T>(E, side == EH_LEFT, 0, ka, side == EH_LEFT ? n : m, alpha, B, ldb, w, s);
   } else {
     const TrsmWork<T> w{base, base + inv, leaf};
     return side == EH_LEFT ? trsm_left<T>(E, 0, m, B, ldb, n, alpha, w, s)

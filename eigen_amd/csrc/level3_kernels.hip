@@ -81,8 +81,8 @@ hipError_t launch_tri_dense(const T* A, int64_t lda, int n, T* D, int64_t ldd, b
 // workgroup of four waves per block: block b is M_b(i, k) = mt ? A[k + i*lda]
 // : A[i + k*lda] at A + b*64 (1 + lda), of order nb = min(64, order - 64 b),
 // lower or upper, unit diagonal or not; its inverse goes to W + b*64*64
-// (ld 64, stored like M: column-major, or row-major when mt; zeros outside the
-// triangle).  Entries of M_b outside
+// (ld 64, stored like M: column-major, or row-major when mt and not columns;
+// zeros outside the triangle).  Entries of M_b outside
 // its triangle and past nb are zero in LDS and the diagonal past nb is one.
 // An upper block is inverted as the lower one its reversed rows and columns
 // form.
@@ -177,8 +177,9 @@ __global__ void __launch_bounds__(256) trtri64_kernel(TrtriParams<T> p) {
 #pragma unroll
   for (int q = 0; q < NB * NB / 256; ++q) {
     const int i = lane, k = w + 4 * q;
-    // p.mt: row i of the inverse is contiguous in W, else column k
-    const int r = p.mt ? k : i, c = p.mt ? i : k;
+    // row-major: row i of the inverse is contiguous in W, else column k
+    const bool rows = p.mt && !p.columns;
+    const int r = rows ? k : i, c = rows ? i : k;
     W[i + k * NB] = rev ? V[NB - 1 - r][NB - 1 - c] : V[r][c];
   }
 }
@@ -371,6 +372,53 @@ hipError_t launch_trsm_panel(const TrsmPanelParams<T>& p, hipStream_t s) {
 }
 template hipError_t launch_trsm_panel<float>(const TrsmPanelParams<float>&, hipStream_t);
 template hipError_t launch_trsm_panel<double>(const TrsmPanelParams<double>&, hipStream_t);
+
+// The panels' off-diagonal 64 x 64 blocks of a triangle with contiguous rows,
+// turned through LDS; workgroup (q, p) takes the q-th pair of blocks of panel p.
+// The panel kernel reads contiguous rows 64 bytes at a time, of sixteen rows at
+// once: FP64 rows a multiple of 128 bytes apart then all want the same halves of
+// their lines, and a panel of 512 takes 54 us instead of 36 (44 at other leading
+// dimensions).  One pass over the panels, each read by every workgroup of 16
+// right-hand sides, costs 3 us for one panel and about 1 for each further:
+// order 8192, 16 right-hand sides, transposed: 1153 -> 870 us.
+template <typename T>
+__global__ void __launch_bounds__(256) turn_panels_kernel(const T* A, int64_t lda, int order, int lower, T* D, int ldd) {
+  constexpr int NB = kTrsmLeaf;
+  __shared__ T tile[NB][NB + 1];
+  int bi = 1, bj = blockIdx.x;  // bi > bj
+  while (bj >= bi) bj -= bi++;
+  if (!lower) {
+    const int t = bi;
+    bi = bj;
+    bj = t;
+  }
+  const int64_t d = (int64_t)blockIdx.y * kTrsmPanel;
+  const int i0 = bi * NB, k0 = bj * NB, sz = (int)min((int64_t)kTrsmPanel, order - d);
+  if (max(i0, k0) >= sz) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  A += d * (1 + lda);
+  D += d * ldd;
+#pragma unroll
+  for (int q = 0; q < NB / 4; ++q) {
+    const int i = w + 4 * q;
+    tile[i][lane] = i0 + i < sz && k0 + lane < sz ? A[k0 + lane + (int64_t)(i0 + i) * lda] : T(0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NB / 4; ++q) {
+    const int k = w + 4 * q;
+    D[i0 + lane + (int64_t)(k0 + k) * ldd] = tile[lane][k];
+  }
+}
+template <typename T>
+hipError_t launch_turn_panels(const T* A, int64_t lda, int order, bool lower, T* D, int ldd, hipStream_t s) {
+  if (order <= kTrsmLeaf) return hipSuccess;
+  const int blocks = (std::min(order, kTrsmPanel) + kTrsmLeaf - 1) / kTrsmLeaf;
+  const dim3 grid((unsigned)(blocks * (blocks - 1) / 2), (unsigned)((order + kTrsmPanel - 1) / kTrsmPanel));
+  hipLaunchKernelGGL(turn_panels_kernel<T>, grid, dim3(256), 0, s, A, lda, order, (int)lower, D, ldd);
+  return hipGetLastError();
+}
+template hipError_t launch_turn_panels<double>(const double*, int64_t, int, bool, double*, int, hipStream_t);
 
 // D (m x n, ld m) = B, lanes along the columns' rows.
 // Eight columns per workgroup and pass, all their loads before the first store

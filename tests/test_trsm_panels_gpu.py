@@ -73,3 +73,15 @@ def test_leading_dimension_past_32_bit_offsets(gpu, trans):
     E.trsm(E.F32, E.LEFT, E.LOWER, E.OP_T if trans else E.OP_N, E.NON_UNIT, ka, n, 1.0, A, lda, dB, ka)
     want = np.linalg.solve((t.T if trans else t).astype(np.float64), B.astype(np.float64))
     assert np.linalg.norm(from_dev(dB, B.shape) - want) <= 8 * ka * 2.0 ** -24 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("ka,other", [(2048, 3), (2049, 5), (2600, 18)])
+def test_halves(gpu, dt, ka, other):
+    """Systems of more than 2048 rows are halved first: every arrangement, a
+    ragged last panel in either half, alpha applied once to both."""
+    rng = np.random.default_rng(ka)
+    for side, lower, trans in itertools.product("LR", (True, False), (False, True)):
+        t, stored = _triangle(rng, ka, dt, lower)
+        m, n = (ka, other) if side == "L" else (other, ka)
+        _check(dt, side, lower, trans, t, stored, ka + 1, m, n, rng)
