@@ -100,7 +100,13 @@ int64_t half(int64_t sz, int64_t leaf) {
 // 107 us.  Systems of more than kTrsmRange rows are halved first, so that most
 // of their work is in products of depth 1024 and more: FP64 8192 x 8192 10.3 ->
 // 9.6 ms (the recursion: 9.8).
+// FP64 systems of two to 64 right-hand sides take panels of half the rows, so
+// that less of the work is on the one to four CUs of the chain (16384, 16 columns
+// 1869 -> 1768 us, 2048, 4 columns 177 -> 167).  One column's updates are
+// matrix-vector products whose launches cost more than that (16384: 1529 ->
+// 1595), as all of FP32's do (2048, 16 columns 128 -> 131).
 constexpr int64_t kTrsmRange = 2048;
+constexpr int64_t kTrsmFew = 64;
 //
 // Complex types: the recursion below.  The diagonal blocks of order
 // kTrsmLeafComplex are inverted up front (one launch); a leaf of the
@@ -149,11 +155,14 @@ eh_status trsm_panels(const Tri<T>& E, bool left, int64_t d0, int64_t size, int6
     EH_TRY(update(d2, n2, d1, n1, alpha));
     return trsm_panels(E, left, d2, n2, other, T(1), B, ldb, w, s);
   }
-  const int64_t np = (size + kTrsmPanel - 1) / kTrsmPanel;
+  const bool few = std::is_same<T, double>::value && other > 1 && other <= kTrsmFew && size > kTrsmPanel;
+  const int64_t panel = few ? kTrsmPanel / 2 : kTrsmPanel;
+  const int64_t np = (size + panel - 1) / panel;
   for (int64_t q = 0; q < np; ++q) {
-    const int64_t d = d0 + (lower ? q : np - 1 - q) * kTrsmPanel, sz = std::min<int64_t>(kTrsmPanel, d0 + size - d);
+    const int64_t d = d0 + (lower ? q : np - 1 - q) * panel, sz = std::min(panel, d0 + size - d);
     TrsmPanelParams<T> p{};
-    p.A = w.turned ? w.turned + d * w.ldt : E.diag(d);
+    const int64_t dp = d % kTrsmPanel;
+    p.A = w.turned ? w.turned + (d - dp) * w.ldt + dp * (1 + w.ldt) : E.diag(d);
     p.inv = w.inv + d * kTrsmLeaf;
     p.B = left ? B + d : B + d * ldb;
     p.lda = w.turned ? w.ldt : E.lda;
