@@ -281,11 +281,13 @@ __global__ void __launch_bounds__(64 * kGemvTWaves, 8) gemv_t_kernel(GemvParams<
 // short ones; gemv_t_kernel spends its two loads per row and the copy of x to
 // LDS on rows that need neither: FP32 500,000 rows of 100 35.4 us (5.6 TB/s)
 // against 80.8, 1,000,000 of 8 63 against 85, FP64 500,000 of 100 71 against 94.
+// Rows that fill the chip two to a wave or not at all run so, since the sums of
+// eight end later: FP32 1000 x 64 3.9 -> 2.4 us, 16,000 x 128 4.4 -> 3.5 (64,000:
+// 7.4 -> 8.9), FP64 1000 x 64 4.0 -> 2.4, 64,000 x 128 14.3 -> 11.3.
 constexpr int kGemvShortRows = 8;
-template <typename T>
+template <typename T, int RW>
 __global__ void __launch_bounds__(256) gemv_t_short_kernel(GemvParams<T> p) {
   constexpr int EPT = 16 / sizeof(T);
-  constexpr int RW = kGemvShortRows;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r0 = (blockIdx.x * 4 + wave) * RW, kl = lane * EPT;
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(p.A, p.bytesA);
@@ -327,7 +329,7 @@ static GemvPlan gemv_t_plan(int m, int k, int es) {
   GemvPlan best{};
   if (k <= chunk) {  // gemv_t_short_kernel
     best.batch = kGemvShortRows;
-    best.rows = 4 * kGemvShortRows;
+    best.rows = 4 * (m <= (es == 8 ? 65536 : 16384) ? 2 : kGemvShortRows);
     best.blocks = (int)(((int64_t)m + best.rows - 1) / best.rows);
     best.splits = 1;
     best.per = k;
@@ -406,7 +408,8 @@ hipError_t launch_gemv(const GemvPlan& g, bool trans, int m, int k, T alpha, con
   const bool short_rows = trans && g.batch == kGemvShortRows;
   const dim3 threads(trans && !short_rows ? 64 * kGemvTWaves : 256);
   if (short_rows) {
-    hipLaunchKernelGGL(gemv_t_short_kernel<T>, grid, threads, 0, s, p);
+    auto k = g.rows == 4 * kGemvShortRows ? gemv_t_short_kernel<T, kGemvShortRows> : gemv_t_short_kernel<T, 2>;
+    hipLaunchKernelGGL(k, grid, threads, 0, s, p);
   } else if (trans) {
     const bool parts = (int64_t)g.per * (int)sizeof(T) > kGemvTBytes;
     auto k = parts          ? (nt ? gemv_t_kernel<T, 1, 8, true, true> : gemv_t_kernel<T, 1, 8, false, true>)

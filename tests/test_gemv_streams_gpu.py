@@ -93,7 +93,7 @@ def test_long_inner_products_exact(gpu, dtype, m, n, incx):
 
 @pytest.mark.parametrize("dtype,code", [(np.float32, E.F32), (np.float64, E.F64)])
 @pytest.mark.parametrize("m", [1, 3, 64, 127, 128, 129, 255, 256, 257])
-@pytest.mark.parametrize("n,pad,incx,incy", [(1, 0, 1, 1), (31, 1, 2, 1), (33, 3, -1, 2), (5000, 0, 1, -1)])
+@pytest.mark.parametrize("n,pad,incx,incy", [(1, 0, 1, 1), (31, 1, 2, 1), (33, 3, -1, 2), (5000, 0, 1, -1), (16385, 1, 1, 1), (65537, 0, 2, 1)])
 def test_gemv_t_short_rows_exact(gpu, dtype, code, m, n, pad, incx, incy):
     """Rows around one 1 KB load of a wave (128 FP64, 256 FP32 elements): each is
     followed by NaN, or by the next row, where it ends."""
