@@ -1,6 +1,7 @@
 """Short driver for profiler runs, and the summariser of their output.
 
-    python3 -m eigen_amd.profile_kernels run {split3,plain,dgemm,batched,dtrsm,zgemm,bf16,copy} [reps] [warmup]
+    python3 -m eigen_amd.profile_kernels run {split3,plain,dgemm,batched,dtrsm,zgemm,bf16,balanced,small,gemv,strided,
+                                              panels,copy} [reps] [warmup]
     python3 -m eigen_amd.profile_kernels summarize <rocprofv3 output root> [traffic.json] [--skip N]
 
 `run` launches one workload `warmup` times (default 2), then `reps` times
@@ -18,6 +19,11 @@ program under `rocprofv3 --kernel-trace --stats` or `rocprofv3 --pmc`:
   dtrsm    dtrsm 8192 x 8192 (left, lower, no transpose), diagonal 2, off-diagonal U[-1/n, 1/n]
   zgemm    zgemm 4096^3 (complex128, one real product over 2x2 real blocks)
   bf16     bf16 inputs, FP32 result, 8192^3 (U[-1,1] rounded to bf16)
+  balanced dgemm 1000x777x1203, A transposed: tiles cut between workgroups
+  small    sgemm 96x80x112, C = 1.5*A*B + 0.5*C
+  gemv     dgemv A^T x, 6000 x 4001
+  strided  20,000 FP64 16x16x16 products at fixed strides
+  panels   dtrsm 1000 x 600 (left, lower, no transpose), operands as dtrsm's
   copy     a 1 GiB device-to-device copy: calibrates the HBM byte counters
 
 `summarize` reads directories named trace_<workload> (kernel-trace csv; with
@@ -45,11 +51,13 @@ COPY_BYTES = 1 << 30
 # dominant kernel of each workload (substring of its name)
 DOMINANT = {"split3": "gemm_split_packed_kernel", "plain": "gemm_mfma_kernel<float", "dgemm": "gemm_mfma_kernel<double",
             "batched": "grouped_gemm_kernel", "dtrsm": "gemm_mfma_kernel<double", "zgemm": "gemm_mfma_kernel<double",
-            "bf16": "gemm_split_packed_kernel", "copy": "copyBuffer"}
+            "bf16": "gemm_split_packed_kernel", "balanced": "gemm_balanced_kernel", "small": "gemm_small_kernel",
+            "gemv": "gemv_t_kernel", "strided": "small_batched_kernel", "panels": "trsm_panel_kernel", "copy": "copyBuffer"}
 
 
 KCLASS = {"split3": "KC_PACKED_PRODUCT", "bf16": "KC_PACKED_PRODUCT", "plain": "KC_PRODUCT", "dgemm": "KC_PRODUCT",
-          "zgemm": "KC_PRODUCT", "dtrsm": "KC_PRODUCT", "batched": "KC_GROUPED"}
+          "zgemm": "KC_PRODUCT", "dtrsm": "KC_PRODUCT", "batched": "KC_GROUPED", "balanced": "KC_PRODUCT", "small": "KC_PRODUCT",
+          "gemv": "KC_GEMV", "strided": "KC_GROUPED"}
 
 
 def run(what: str, reps: int, warmup: int = 2) -> None:
@@ -103,14 +111,14 @@ def _workload(E, torch, what: str):
         b = uneven_batch(20000, seed=0)
         g = E.Grouped(b.problems)
         return lambda: (g.run(), b)  # b owns the operand buffers
-    elif what == "dtrsm":
-        n = 8192
+    elif what in ("dtrsm", "panels"):
+        n, cols = (8192, 8192) if what == "dtrsm" else (1000, 600)
         A = torch.empty(n * n, dtype=torch.float64, device="cuda")
-        B = torch.empty(n * n, dtype=torch.float64, device="cuda")
+        B = torch.empty(n * cols, dtype=torch.float64, device="cuda")
         E.fill(E.F64, A, n * n, 31, E.DIST_UNIFORM, -1.0 / n, 1.0 / n)
         A.view(n, n).diagonal().fill_(2.0)
-        E.fill(E.F64, B, n * n, 32, E.DIST_UNIFORM, -1, 1)
-        return lambda: E.trsm(E.F64, E.LEFT, E.LOWER, E.OP_N, E.NON_UNIT, n, n, 1.0, A, n, B, n)
+        E.fill(E.F64, B, n * cols, 32, E.DIST_UNIFORM, -1, 1)
+        return lambda: E.trsm(E.F64, E.LEFT, E.LOWER, E.OP_N, E.NON_UNIT, n, cols, 1.0, A, n, B, n)
     elif what == "zgemm":
         n = 4096
         A, B, Cm = (torch.rand(2 * n * n, dtype=torch.float64, device="cuda") * 2 - 1 for _ in range(3))
@@ -121,6 +129,22 @@ def _workload(E, torch, what: str):
         B = (torch.rand(n * n, device="cuda") * 2 - 1).to(torch.bfloat16)
         Cm = torch.zeros(n * n, device="cuda")
         return lambda: E.gemm_bf16(0, 0, n, n, n, 1.0, A.data_ptr(), n, B.data_ptr(), n, 0.0, Cm, n)
+    elif what in ("balanced", "small"):
+        f64 = what == "balanced"
+        m, n, k = (1000, 777, 1203) if f64 else (96, 80, 112)
+        A, B, Cm = (torch.rand(q, dtype=torch.float64 if f64 else torch.float32, device="cuda") * 2 - 1
+                    for q in (m * k, k * n, m * n))
+        if f64:
+            return lambda: E.gemm(E.F64, 1, 0, m, n, k, 1.0, A, k, B, k, 0.0, Cm, m)
+        return lambda: E.gemm(E.F32, 0, 0, m, n, k, 1.5, A, m, B, k, 0.5, Cm, m, prec=E.PREC_PLAIN)
+    elif what == "gemv":
+        m, n = 6000, 4001
+        A, x, y = (torch.rand(q, dtype=torch.float64, device="cuda") * 2 - 1 for q in (m * n, m, n))
+        return lambda: E.gemv(E.F64, 1, m, n, 1.0, A, m, x, 1, 0.0, y, 1)
+    elif what == "strided":
+        count = 20000
+        A, B, Cm = (torch.rand(256 * count, dtype=torch.float64, device="cuda") * 2 - 1 for _ in range(3))
+        return lambda: E.gemm_batched_strided(E.F64, 0, 0, 16, 16, 16, 1.0, A, 16, 256, B, 16, 256, 0.0, Cm, 16, 256, count)
     elif what == "copy":
         x = torch.empty(COPY_BYTES // 4, dtype=torch.float32, device="cuda")
         y = torch.empty_like(x)
