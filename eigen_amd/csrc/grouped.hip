@@ -47,7 +47,7 @@
 // the device, except for small shapes, which take kernels of their own: up
 // to 4 x 4 x 4 one thread per product (whole-column accesses for dense
 // 2 x 2 and 4 x 4 matrices, nine-element runs for dense 3 x 3 ones), up to
-// 16 x 16 with depth up to 64 (FP64) or 32 (FP32) one wave per product.
+// 32 x 32 with depth up to 64 one wave per product.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

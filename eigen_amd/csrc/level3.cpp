@@ -97,7 +97,7 @@ int64_t half(int64_t sz, int64_t leaf) {
 // still to be solved.  Two launches per panel replace the recursion's one
 // product per block and level with a copy of every block: order 1000 with
 // 600 right-hand sides in FP64 took 58 launches and 372 us, against 5 and
-// 107 us.  Systems of more than kTrsmRange rows are halved first, so that most
+// 110 us.  Systems of more than kTrsmRange rows are halved first, so that most
 // of their work is in products of depth 1024 and more: FP64 8192 x 8192 10.3 ->
 // 9.6 ms (the recursion: 9.8).
 // FP64 systems of two to 64 right-hand sides take panels of half the rows, so
@@ -107,7 +107,7 @@ int64_t half(int64_t sz, int64_t leaf) {
 // 1595), as all of FP32's do (2048, 16 columns 128 -> 131).
 constexpr int64_t kTrsmRange = 2048;
 constexpr int64_t kTrsmFew = 64;
-//
+
 // Complex types: the recursion below.  The diagonal blocks of order
 // kTrsmLeafComplex are inverted up front (one launch); a leaf of the
 // recursion multiplies its right-hand sides by the inverse of its block, on
@@ -240,7 +240,7 @@ eh_status trsm_right(const Tri<T>& E, int64_t d, int64_t sz, T* B, int64_t ldb, 
 // ---- TRMM --------------------------------------------------------------------
 // Real types: ranges up to kTrmmLeafReal multiply a copy of their part of B
 // by the triangle itself in one launch (tri_product).  FP32 1500 x 1100 from
-// the right: 48 us, against 180 through 256-row dense leaves (17 launches);
+// the right: 51 us, against 180 through 256-row dense leaves (17 launches);
 // FP64 8192 x 8192: 9.3 against 9.9 ms.
 // Complex types, and triangles past 32-bit addressing, expand dense leaves.
 constexpr int64_t kTrmmLeaf = 256;
