@@ -160,14 +160,20 @@ static eh_precision default_sgemm_precision() {
 // stream queue their launch sequences one after another.  Growing replaces
 // the buffer; the old one is freed when its last reference goes, with
 // hipFree, which waits for the device, so work queued with it completes
-// before the memory is released.  A buffer that a captured call was given
-// stays allocated, since the graph holds its address and may be replayed at
-// any time; its successor is at least twice its size, so that all of a
-// stream's kept buffers together are smaller than the present one.
+// before the memory is released.
+//
+// Captured calls have buffers of their own: a graph holds its buffer's address
+// and may be replayed at any time and on any stream, beside eager calls on the
+// stream it was captured on, so its buffer is neither freed nor given to those.
+// The first captured call takes over the buffer that eager calls have grown so
+// far (nothing can be allocated then), and the next eager call starts a new
+// one.  Later captures on the stream share that buffer; one that needs more
+// takes over the eager buffer again.  From then on sizes are powers of two, so
+// all of a stream's kept buffers together are below twice the largest.
 struct WorkspaceSlot {
   std::recursive_mutex mu;
-  std::shared_ptr<Workspace> buf;
-  std::vector<std::shared_ptr<Workspace>> captured;
+  std::shared_ptr<Workspace> buf;                   // eager calls
+  std::vector<std::shared_ptr<Workspace>> graphs;  // captured calls: the last one serves the next
 };
 static std::map<std::tuple<int, hipStream_t, std::thread::id>, std::unique_ptr<WorkspaceSlot>> g_ws;
 
@@ -234,8 +240,12 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
   }
   WorkspaceLease lease;
   lease.lock = std::unique_lock<std::recursive_mutex>(slot->mu);
-  if (!slot->buf || slot->buf->bytes < bytes) {
-    const size_t have = slot->buf ? slot->buf->bytes : 0;
+  const bool capturing = stream_capturing(stream);
+  if (capturing && slot->buf && slot->buf->bytes >= bytes &&
+      (slot->graphs.empty() || slot->graphs.back()->bytes < bytes))
+    slot->graphs.push_back(std::move(slot->buf));
+  std::shared_ptr<Workspace> cur = !capturing ? slot->buf : slot->graphs.empty() ? nullptr : slot->graphs.back();
+  if (!cur || cur->bytes < bytes) {
     // hipMalloc and hipFree end every capture in progress, on any stream,
     // unless the calling thread's mode says that it does not mean them to
     struct RelaxedCapture {
@@ -245,12 +255,13 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
       ~RelaxedCapture() {
         if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
       }
-    } relaxed(!stream_capturing(stream));
-    const bool keep = slot->buf && slot->buf->captured;
+    } relaxed(!capturing);
+    size_t want = std::max(bytes, std::max(cur ? cur->bytes : 0, (size_t)1 << 20));
+    if (!slot->graphs.empty())
+      while (want & (want - 1)) want += want & -want;  // up to a power of two
     auto fresh = std::make_shared<Workspace>();
-    const size_t want = std::max(bytes, std::max(keep ? 2 * have : have, (size_t)1 << 20));
-    if (keep) slot->captured.push_back(std::move(slot->buf));
-    slot->buf.reset();  // any other old buffer goes once no lease refers to it
+    cur.reset();
+    if (!capturing) slot->buf.reset();  // the old buffer goes once no lease refers to it
     e = hipMalloc(&fresh->base, want + kTicketBytes);
     if (e != hipSuccess) {
       fresh->base = nullptr;
@@ -258,10 +269,13 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
     }
     fresh->ptr = static_cast<unsigned char*>(fresh->base) + kTicketBytes;
     fresh->bytes = want;
-    slot->buf = std::move(fresh);
+    cur = fresh;
+    if (capturing)
+      slot->graphs.push_back(std::move(fresh));
+    else
+      slot->buf = std::move(fresh);
   }
-  lease.buf = slot->buf;
-  lease.buf->captured |= stream_capturing(stream);
+  lease.buf = std::move(cur);
   *ptr = lease.buf->ptr;
   *out = std::move(lease);
   return EH_SUCCESS;

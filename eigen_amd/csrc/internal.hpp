@@ -50,7 +50,6 @@ struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
   bool tickets_clear = false;
-  bool captured = false;  // a graph may hold its address
   Workspace() = default;
   Workspace(const Workspace&) = delete;
   Workspace& operator=(const Workspace&) = delete;

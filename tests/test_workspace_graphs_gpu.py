@@ -76,3 +76,29 @@ def test_eager_call_beside_a_capture(gpu, before):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(c, want)
+
+
+def test_replay_beside_eager_calls(gpu):
+    """A graph replayed on another stream while the stream it was captured on
+    runs products that need workspace: each keeps its own partial sums."""
+    small, big = (130, 130, 20000), (1000, 777, 1203)
+    ab, want = operands(*small, 1)
+    bab, bwant = operands(*big, 3)
+    c, bc = torch.zeros_like(want), torch.zeros_like(bwant)
+    s, r, g = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        product(*small, ab, c, s)
+        torch.cuda.synchronize()
+        g.capture_begin()
+        product(*small, ab, c, s)
+        g.capture_end()
+    for _ in range(30):
+        c.zero_(), bc.zero_()
+        torch.cuda.synchronize()
+        for _ in range(4):
+            with torch.cuda.stream(r):
+                g.replay()
+            product(*big, bab, bc, s)
+        torch.cuda.synchronize()
+        assert torch.equal(c, want) and torch.equal(bc, bwant)
