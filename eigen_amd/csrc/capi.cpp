@@ -152,6 +152,8 @@ static eh_precision default_sgemm_precision() {
 }
 
 // ---- workspace --------------------------------------------------------------
+constexpr size_t kWorkspaceMin = 1 << 20;
+
 // One growable device buffer per (device, stream) for split-K partials, packed
 // operands and work lists; hipStreamPerThread names a different stream in
 // every thread, so it is keyed per thread as well.  A call holds the stream's
@@ -256,7 +258,7 @@ eh_status workspace_get(hipStream_t stream, size_t bytes, WorkspaceLease* out, v
         if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
       }
     } relaxed(!capturing);
-    size_t want = std::max(bytes, std::max(cur ? cur->bytes : 0, (size_t)1 << 20));
+    size_t want = std::max(bytes, std::max(cur ? cur->bytes : 0, kWorkspaceMin));
     if (!slot->graphs.empty())
       while (want & (want - 1)) want += want & -want;  // up to a power of two
     auto fresh = std::make_shared<Workspace>();
@@ -761,7 +763,20 @@ eh_status complex_a_product(bool ta, bool conj, int64_t m, int64_t n, int64_t k,
   p.bytesA = (uint32_t)((ta ? (uint64_t)(m - 1) * lda + k : (uint64_t)(k - 1) * lda + m) * 2 * sizeof(T));
   p.alpha_im = ai;
   p.conj = conj;
-  return launch_balanced<T>(p, kComplexA, ta, false, stream);
+  // the workspace grows to what the planner's product needs too (run_gemm); not
+  // planned where the slots hold any split of it
+  size_t need = (size_t)8 * 2 * m * n * sizeof(T);
+  const int64_t b = kBalancedTile, bk = 128 / (int64_t)sizeof(T);
+  const int64_t tiles = ((2 * m + b - 1) / b) * ((n + b - 1) / b);
+  const size_t slots = (size_t)balanced_groups(tiles * ((2 * k + bk - 1) / bk)) * 2 * b * b * sizeof(T);
+  if (need > std::max(slots, kWorkspaceMin)) {
+    int config = 0, tile = 0, splits = 1;
+    eh_status st = plan_config(std::is_same<T, double>::value ? EH_F64 : EH_F32, EH_OP_N, EH_OP_N, 2 * m, n, 2 * k, &config);
+    if (st != EH_SUCCESS) return st;
+    config_decode(config, &tile, &splits);
+    need = splits > 1 ? need / 8 * splits : 0;
+  }
+  return launch_balanced<T>(p, kComplexA, ta, false, stream, need);
 }
 template eh_status complex_a_product<float>(bool, bool, int64_t, int64_t, int64_t, float, float, const float*, int64_t,
                                             const float*, int64_t, float, float*, int64_t, hipStream_t);

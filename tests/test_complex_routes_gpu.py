@@ -84,3 +84,27 @@ def test_few_tiles(gpu):
     """Two tiles of deep k: in place, one workgroup would add 64 parts each."""
     c, want = both(*operands(3, 64, 64, 2048))
     assert torch.equal(c, want)
+
+
+def test_captured_after_one_eager_call(gpu):
+    """The eager call, in place, grows the stream's workspace to what the captured
+    one's split K needs (145 MB; its own slots take 48)."""
+    m, n, k = 1603, 1483, 1537
+    a, b, a3 = operands(4, m, n, k)
+    assert E.config_info(E.plan(E.F64, 0, 0, 2 * m, n, 2 * k))[2] > 1
+    c, s, g = torch.zeros(n, m, dtype=torch.complex128, device="cuda"), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    want = (b @ a).contiguous()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        complex_product(a, b, c, s.cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.allclose(c, want, rtol=0, atol=1e-11)
+        g.capture_begin()
+        complex_product(a, b, c, s.cuda_stream)
+        g.capture_end()
+    for _ in range(2):
+        c.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.allclose(c, want, rtol=0, atol=1e-11)
